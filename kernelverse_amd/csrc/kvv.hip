@@ -840,6 +840,7 @@ int run_single(const SegDesc& d0, kvv_result* out, void* ws, size_t ws_bytes, hi
   if (d.item_count > 0) {
     ScanArgs a = g.rounds;
     a.seg0 = d;
+    a.rows0 = row_map(d);
     a.table = nullptr;
     a.nseg = 1;
     a.item_lo = 0;

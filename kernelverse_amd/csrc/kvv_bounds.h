@@ -30,4 +30,14 @@ KVV_HD inline CellSpan cell_span(uint32_t t_lo, uint32_t t_hi, int64_t count, in
   return CellSpan{lo, len};
 }
 
+// floor(x / d) for every x < 2^31 (2 <= d < 2^31) as mulhi(x, mul) >> sh: with l
+// = ceil(log2 d), mul = floor(2^(31 + l) / d) + 1 fits 32 bits, mul * d exceeds
+// 2^(31 + l) by at most d <= 2^l, and x * 2^l < 2^(31 + l), so the quotient is exact.
+KVV_HD inline void row_magic(uint32_t d, uint32_t& mul, uint32_t& sh) {
+  uint32_t l = 1;
+  while (l < 31 && (1u << l) < d) ++l;
+  mul = (uint32_t)((1ull << (31 + l)) / d + 1);
+  sh = l - 1;
+}
+
 }  // namespace kvv

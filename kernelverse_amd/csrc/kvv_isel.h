@@ -322,37 +322,22 @@ static_assert(kPivotSamples == 16 * kBlock && kPivotRun == 64 && kSmall < kIselC
               "pivot values: 16 per thread, one run per wave and step, fewer than a capture segment's");
 
 // Capture thresholds.  A NaN among the pivot values (the p99 is then NaN)
-// captures the NaNs only.  cap_rel_lo and cap_rel_hi bound where rel_diff =
-// fl(abs_diff / den), den = fl(|ref| + 1e-12), reaches cap_key[1] without the
-// division (the threshold value v, u = 2^-24 the rounding unit):
-// * below: abs_diff < fl(cap_rel_lo * den) gives fl(abs_diff / den) < v,
-//   since cap_rel_lo <= v * (1 - 2^-20) and every product stays a normal float
-//   (v >= 2^-80, den >= 1e-12; larger v are capped at 2^127, past which only
-//   the division tells).  fl(cap_rel_lo * |ref|) is never above that product.
-// * above: abs_diff >= H = fl(cap_rel_hi * |ref| + cap_rel_hic), with
-//   cap_rel_hi = fl(v * (1 + 2^-20)) and cap_rel_hic = fl(cap_rel_hi * 1e-12),
-//   gives H >= cap_rel_hi * (|ref| + 1e-12) * (1 - u)^2 >= cap_rel_hi * den *
-//   (1 - u)^3, so abs_diff / den > v * (1 + 2^-20) * (1 - u)^4 > v and the
-//   rounded quotient is at least v.  Taken for 2^-80 <= v < 2^100 (products
-//   normal or, where they overflow, H infinite and the test false); else
-//   cap_rel_hi is +inf and only the division tells.
+// captures the NaNs only.  cap_rel_lo bounds where rel_diff = fl(abs_diff /
+// den), den = fl(|ref| + 1e-12), can reach cap_key[1] without the division (the
+// threshold value v): abs_diff < fl(cap_rel_lo * den) gives fl(abs_diff / den)
+// < v, since cap_rel_lo <= v * (1 - 2^-20) and every product stays a normal
+// float (v >= 2^-80, den >= 1e-12; larger v are capped at 2^127, past which
+// only the division tells).  fl(cap_rel_lo * |ref|) is never above that product.
 __device__ inline void set_thresholds(SegDesc& d, uint32_t ka, bool nan_a, uint32_t kr, bool nan_r) {
   const uint32_t k0 = nan_a ? 0xFFFFFFFFu : ka, k1 = nan_r ? 0xFFFFFFFFu : kr;
   d.cap_key[0] = k0 > kZeroKey ? k0 : kZeroKey + 1u;
   d.cap_key[1] = k1 > kZeroKey ? k1 : kZeroKey + 1u;
   const float v = fkey_value(d.cap_key[1]);
-  float lo, hi = __builtin_inff();
-  if (d.cap_key[1] == 0xFFFFFFFFu) {
-    lo = __builtin_inff();
-  } else if (v < 0x1p-80f) {
-    lo = 0.0f;
-  } else {
-    lo = fminf(v * (1.0f - 0x1p-20f), 0x1p127f);
-    if (v < 0x1p100f) hi = v * (1.0f + 0x1p-20f);
-  }
+  float lo;
+  if (d.cap_key[1] == 0xFFFFFFFFu) lo = __builtin_inff();
+  else if (v < 0x1p-80f) lo = 0.0f;
+  else lo = fminf(v * (1.0f - 0x1p-20f), 0x1p127f);
   d.cap_rel_lo = lo;
-  d.cap_rel_hi = hi;
-  d.cap_rel_hic = hi * 1e-12f;
 }
 
 // Counts of bins [tid * 8, tid * 8 + 8) of both block histograms.
@@ -767,14 +752,16 @@ __global__ __launch_bounds__(kBlock) void isel_cap_final_kernel(IselArgs a) {
   const bool nan[2] = {st[IS_CNAN] != 0, st[IS_CNAN + 1] != 0};
   const CapRanks c0 = cap_ranks(d, cap[0], st[IS_BELOW], nan[0], rank64);
   const CapRanks c1 = cap_ranks(d, cap[1], st[IS_BELOW + 1], nan[1], rank64);
-  if (st[IS_CNEG] != 0 || c0.miss || c1.miss) {
-    // the fallback takes the segment over, from cleared histograms and counts
-    // (not the words either block reads above)
-    if (x != 0) return;
+  // the fallback takes the segment over, from cleared histograms and counts
+  // (not the words either block reads above)
+  auto fall_back = [&]() {
     __syncthreads();
     for (int i = tid; i <= IS_BASE + 3; i += kBlock)
       if (i != IS_FILL && i != IS_FILL + 1) st[i] = 0;
     if (tid == 0) a.fb_segs[atomicAdd(a.fb_scount, 1u)] = seg;
+  };
+  if (st[IS_CNEG] != 0 || c0.miss || c1.miss) {
+    if (x == 0) fall_back();
     return;
   }
   const CapRanks& c = x == 0 ? c0 : c1;
@@ -784,6 +771,13 @@ __global__ __launch_bounds__(kBlock) void isel_cap_final_kernel(IselArgs a) {
     const uint32_t r2[2] = {c.need[0] ? c.rk[0] : c.rk[1], c.need[1] ? c.rk[1] : c.rk[0]};
     uint32_t k[2];
     range_keys(a.buf[x] + d.sample_off, cap[x], r2, k, L);
+    // The main pass's dense items capture rel_diff from cap_rel_lo on, a few
+    // roundings below the threshold: an order statistic from the threshold on
+    // has every value that was not captured below it, a lower one may not
+    if (x == 1 && (k[0] < d.cap_key[1] || k[1] < d.cap_key[1])) {
+      fall_back();
+      return;
+    }
     if (c.need[0]) key[0] = k[0];
     if (c.need[1]) key[1] = k[1];
   }

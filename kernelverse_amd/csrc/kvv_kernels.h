@@ -159,10 +159,7 @@ struct SegDesc {
   uint32_t* cap_state;    // the segment's input-select state words
   uint32_t cap_key[2];    // capture the nonzero values whose key is at least these (abs, rel)
   float cap_rel_lo;       // rel_diff can reach cap_key[1] only where abs_diff >= cap_rel_lo * den
-  float cap_rel_hi;       // rel_diff reaches cap_key[1] where abs_diff >= fma(cap_rel_hi, |ref|, cap_rel_hic)
-  float cap_rel_hic;
   int32_t isel_group;     // input-select: the segment's dtype group (which fallback launch takes it)
-  int32_t isel_pad[2];
 };
 
 // Samples per input-select chunk of segment d.
@@ -264,6 +261,9 @@ struct Acc {
   uint32_t nmm;            // mismatches
   uint32_t nnear_fast;     // ... of which near zero
   float rel_thr;           // rel-max filter: only rel >= ~rel_thr can still win
+  // the wave's largest so far (wave-uniform; for the dense path's bounds): rel_diff seen by slow_elem, abs_diff seen
+  // by phase_dense
+  float rel_best, abs_best;
   // element indices are offsets from the run's first element (a run spans
   // fewer than 2^32 - 1 elements), kNone32 for none
   uint32_t first_mm, first_viol;
@@ -276,6 +276,8 @@ struct Acc {
     gabs_k = grel_k = 0;
     nfast = nnear_fast = nmm = 0;
     rel_thr = -__builtin_inff();
+    rel_best = -__builtin_inff();
+    abs_best = -1.0f;
     first_mm = first_viol = kNone32;
     gabs_i = grel_i = kNone32;
     first_fast = kNone32;
@@ -287,11 +289,23 @@ struct Acc {
 
 __device__ __forceinline__ int lane_id() { return (int)(threadIdx.x & 63); }
 
+#define KVV_LDS __attribute__((address_space(3)))
+
+// The dense path's ULP-bucket counters: kRep copies of each bucket's counter
+// per wave (lane l adds to copy l mod kRep, so that at most four lanes of a
+// step meet at an address), bucket b in row kBuckets - 1 - b.
+constexpr int kRep = 16;
+__device__ __forceinline__ int rep_at(int bucket) {
+  return (kBuckets - 1 - bucket) * kRep + (lane_id() & (kRep - 1));
+}
+
 // Wave-uniform values, stated as such so that they live in scalar registers.
 __device__ __forceinline__ uint32_t uniform(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
 __device__ __forceinline__ uint64_t uniform(uint64_t v) {
   return (uint64_t)uniform((uint32_t)v) | ((uint64_t)uniform((uint32_t)(v >> 32)) << 32);
 }
+
+__device__ __forceinline__ float uniform(float v) { return __uint_as_float(uniform(__float_as_uint(v))); }
 
 // Adds the number of lanes where `pred` holds to a per-wave LDS counter
 // (one ds_add by one lane, whatever the number of lanes).
@@ -393,6 +407,15 @@ __device__ __forceinline__ float wave_max_f32(float v) {
   return v;
 }
 
+// The wave's largest rel_diff so far becomes that of its lanes' `best` (NaN the
+// largest of all); called by every active lane.
+__device__ __forceinline__ void raise_rel(Acc& acc, float best) {
+  const bool nan = __ballot(best != best) != 0;
+  const float b = nan ? __builtin_nanf("") : uniform(wave_max_f32(best));
+  acc.rel_best = b;
+  acc.rel_thr = uniform(rel_threshold(b));
+}
+
 // ------------------------------------------------------------ capture (kFlagCapture)
 // A run of items (one wave's, within one segment) writes its captured values
 // compacted into its own elements' part of the segment's sample region: from
@@ -460,16 +483,21 @@ __device__ __forceinline__ void capture_elem(const SegDesc& d, float adf, float 
 
 // Full treatment of one element for the lanes with `act` set.  Every lane of
 // the wave calls it (it uses ballots); counts go to the wave's LDS row `wc`.
-template <int DT, int MODE>
+// With REST, the element's ULP bucket, fp64 products, captured
+// values and near-zero count were already taken with those of its item
+// (phase_dense): what is left are the tests of a mismatch, a rel argmax
+// candidate or a non-finite value, and the bucket of a NaN pair is taken back
+// from the replicated counters `rep`.
+template <int DT, int MODE, bool REST = false>
 __device__ __forceinline__ void slow_elem(typename Elem<DT>::T gc, typename Elem<DT>::T rc, bool act, uint32_t idx,
-                                          const SegDesc& d, Acc& acc, uint32_t* wc) {
+                                          const SegDesc& d, Acc& acc, uint32_t* wc, KVV_LDS uint32_t* rep = nullptr) {
   using E = Elem<DT>;
   float adf, rf;
   uint32_t abs_key;
   bool mm;
   elem_test<DT, MODE>(gc, rc, d, adf, abs_key, mm, rf);
   const float den = fabsf(rf) + 1e-12f;
-  if (d.flags & kFlagCaptureElems) capture_elem(d, adf, den, act, wc);
+  if (!REST && (d.flags & kFlagCaptureElems)) capture_elem(d, adf, den, act, wc);
   mm = mm && act;
   acc.nmm += mm ? 1u : 0u;
   if (mm) {
@@ -486,18 +514,18 @@ __device__ __forceinline__ void slow_elem(typename Elem<DT>::T gc, typename Elem
   // rel argmax: an element below the wave's best so far cannot be the argmax,
   // so the bound is shared by the wave's lanes (the division is then rare)
   bool raised = false;
+  float best = acc.rel_best;
   if (act && !(adf < acc.rel_thr * den)) {
     const float rel = adf / den;
     const uint32_t rk = fkey(rel);
     if (better32(rk, idx, acc.grel_k, acc.grel_i)) {
       acc.grel_k = rk;
       acc.grel_i = idx;
-      const float t = rel_threshold(rel);
-      raised = !(t <= acc.rel_thr);
-      acc.rel_thr = raised ? t : acc.rel_thr;
+      raised = !(rel <= acc.rel_best) && acc.rel_best == acc.rel_best;  // (nothing exceeds a NaN)
+      best = raised ? rel : best;
     }
   }
-  if (__ballot(raised)) acc.rel_thr = wave_max_f32(acc.rel_thr);
+  if (__ballot(raised)) raise_rel(acc, best);
   bool nan_pair = false;
   if constexpr (E::is_float) {
     const bool nf = act && !(E::finite(gc) && E::finite(rc));
@@ -517,37 +545,47 @@ __device__ __forceinline__ void slow_elem(typename Elem<DT>::T gc, typename Elem
       wave_add(wc, LC_NINF_R, nf && ir && E::sign(rc));
       nan_pair = ng || nr;
       wave_add(wc, LC_NANPAIR, act && nan_pair);
+      if constexpr (REST) {
+        if (nf && nan_pair) atomicAdd((uint32_t*)(rep + rep_at(pair_bucket<DT>(gc, rc))), ~0u);
+        if (d.flags & kFlagCaptureElems) {
+          // (a NaN among the captured values makes the quantile NaN, whatever the counts)
+          cap_nan(d, 0, nf && adf != adf);
+          cap_nan(d, 1, nf && adf / den != adf / den);
+        }
+      }
     }
   }
-  // ULP histogram: one aggregated add when the wave's elements share a bucket
-  // (e.g. 1-ULP steps), else every lane adds its own in one LDS atomic
-  // instruction (a loop over the distinct buckets would serialise the wave)
-  const bool hv = act && !nan_pair;
-  const int bk = pair_bucket<DT>(gc, rc);
-  const uint64_t hb = __ballot(hv);
-  if (hb) {
-    const int l0 = __ffsll((long long)hb) - 1;
-    const int kb = __builtin_amdgcn_readlane(bk, l0);  // l0 is wave-uniform: a register read, no LDS trip
-    const uint64_t same = __ballot(hv && bk == kb);
-    if (same == hb) {
-      if (lane_id() == l0) atomicAdd(&wc[LC_HIST0 + kb], (uint32_t)__popcll(same));
-    } else if (hv) {
-      atomicAdd(&wc[LC_HIST0 + bk], 1u);
+  if constexpr (!REST) {
+    // ULP histogram: one aggregated add when the wave's elements share a bucket
+    // (e.g. 1-ULP steps), else every lane adds its own in one LDS atomic
+    // instruction (a loop over the distinct buckets would serialise the wave)
+    const bool hv = act && !nan_pair;
+    const int bk = pair_bucket<DT>(gc, rc);
+    const uint64_t hb = __ballot(hv);
+    if (hb) {
+      const int l0 = __ffsll((long long)hb) - 1;
+      const int kb = __builtin_amdgcn_readlane(bk, l0);  // l0 is wave-uniform: a register read, no LDS trip
+      const uint64_t same = __ballot(hv && bk == kb);
+      if (same == hb) {
+        if (lane_id() == l0) atomicAdd(&wc[LC_HIST0 + kb], (uint32_t)__popcll(same));
+      } else if (hv) {
+        atomicAdd(&wc[LC_HIST0 + bk], 1u);
+      }
     }
-  }
-  if (act) {
-    const double g64 = E::f64(gc), r64 = E::f64(rc);
-    const double d64 = g64 - r64;
-    acc.s[0] = fma(g64, g64, acc.s[0]);
-    acc.s[1] = fma(r64, r64, acc.s[1]);
-    acc.s[2] = fma(g64, r64, acc.s[2]);
-    acc.s[3] = fma(d64, d64, acc.s[3]);
+    if (act) {
+      const double g64 = E::f64(gc), r64 = E::f64(rc);
+      const double d64 = g64 - r64;
+      acc.s[0] = fma(g64, g64, acc.s[0]);
+      acc.s[1] = fma(r64, r64, acc.s[1]);
+      acc.s[2] = fma(g64, r64, acc.s[2]);
+      acc.s[3] = fma(d64, d64, acc.s[3]);
+    }
   }
   if (d.flags & kFlagNearAny) {
     const bool near = fabsf(rf) <= d.nz_abs;
     // (with near-zero entries, every element's near-zero count comes from the item's masks)
-    if (d.flags & KVV_FLAG_NEAR_ZERO) wave_add(wc, LC_NEAR, act && near);
-    wave_add(wc, LC_NEARBAD, act && near && adf > d.nz_bad);
+    if (!REST && (d.flags & KVV_FLAG_NEAR_ZERO)) wave_add(wc, LC_NEAR, act && near);
+    if (!REST) wave_add(wc, LC_NEARBAD, act && near && adf > d.nz_bad);
     wave_add(wc, LC_FARMM, mm && !near);
   }
 }
@@ -616,7 +654,6 @@ __device__ __forceinline__ uint4 nt_load16(const void* p) {
 // ds_read instructions.  Through a generic pointer the compiler may merge an
 // LDS read and a global read of the same value into one flat load, whose wait
 // also waits for the next item's loads in flight.
-#define KVV_LDS __attribute__((address_space(3)))
 typedef const KVV_LDS uint4* StageP;
 
 template <typename T>
@@ -654,6 +691,22 @@ __device__ __forceinline__ uint32_t load_item(const SegDesc& d, int64_t L0, int6
   using T = typename IO::T;
   constexpr int V = IO::V;
   uint32_t full = 0;
+  if constexpr (KIND == K_CONTIG) {
+    if (L1 - L0 == (int64_t)kUnroll * 64 * V) {
+      // a whole item: one scalar base per tensor, the lane's offset and
+      // immediates (no address arithmetic or bounds per lane and vector, which
+      // took about 50 of the 650 VALU instructions of a mostly identical item)
+      const char* pg = reinterpret_cast<const char*>(d.g) + L0 * (int64_t)sizeof(T);
+      const char* pr = reinterpret_cast<const char*>(d.r) + L0 * (int64_t)sizeof(T);
+      const uint32_t off = (uint32_t)lane_id() * 16u;
+#pragma unroll
+      for (int u = 0; u < kUnroll; ++u) {
+        gv[u] = nt_load16(pg + off + u * 1024);
+        rv[u] = nt_load16(pr + off + u * 1024);
+      }
+      return (1u << kUnroll) - 1;
+    }
+  }
   if constexpr (KIND == K_ROWS) {
     if (d.row_items > 0) {
       // every vector of the item lies in row rc.row (no partial vectors: n is whole items)
@@ -1175,13 +1228,11 @@ __device__ __forceinline__ PhaseA phase_a_dot(const SegDesc& d, StageP stage, ui
 // without writing anything; queue_part then appends the slots [p0, p0 + slots)
 // of every lane.
 constexpr int kQSlots = 16;
-constexpr int kRep = 16;  // copies of each ULP bucket counter of the dense path
 template <int DT>
 struct QueueGeom {
   static constexpr bool wide = VecIO<DT>::NE <= 16;
   static constexpr int slots = wide ? kQSlots / 2 : kQSlots;
-  static constexpr int rep_words = wide ? kBuckets * kRep : 1;
-  static_assert(!wide || 64 * slots * 2 >= kBuckets * kRep * 4, "the counters take the queue's other half");
+  static constexpr int rep_words = DT == KVV_F32 || DT == KVV_BF16 || DT == KVV_F16 ? kBuckets * kRep : 1;
 };
 
 template <int SLOTS>
@@ -1214,10 +1265,12 @@ __device__ __forceinline__ uint32_t queue_part(uint32_t part, int p0, uint16_t* 
   return total;
 }
 
-// Phase B: the wave's queued elements, 64 at a time, from the LDS stage.
-template <int DT, int MODE>
+// Phase B: the wave's queued elements, 64 at a time, from the LDS stage (REST:
+// those that a dense item leaves, slow_elem).
+template <int DT, int MODE, bool REST = false>
 __device__ __forceinline__ void phase_b(const SegDesc& d, uint32_t R0, uint32_t total, StageP stage,
-                                        const uint16_t* queue, Acc& acc, uint32_t* wc) {
+                                        const uint16_t* queue, Acc& acc, uint32_t* wc,
+                                        KVV_LDS uint32_t* rep = nullptr) {
   using IO = VecIO<DT>;
   using T = typename IO::T;
   constexpr int V = IO::V;
@@ -1235,7 +1288,7 @@ __device__ __forceinline__ void phase_b(const SegDesc& d, uint32_t R0, uint32_t 
     const T gc = stage_elem<T>(stage, (2 * u) * 64 + src, e);
     const T rc = stage_elem<T>(stage, (2 * u + 1) * 64 + src, e);
     const uint32_t idx = R0 + (uint32_t)((u * 64 + src) * V + e);
-    slow_elem<DT, MODE>(gc, rc, act, idx, d, acc, wc);
+    slow_elem<DT, MODE, REST>(gc, rc, act, idx, d, acc, wc, rep);
   }
 }
 
@@ -1270,36 +1323,43 @@ __device__ __forceinline__ bool phase_b_dense(const SegDesc& d, uint32_t R0, uin
   }
 }
 
-// Phase B in place for an fp32 item of mostly slow pairs under the isclose test
-// without near-zero diagnostics (e.g. every pair perturbed by noise): each lane
-// walks its own slots once and finishes every slow pair whose values have one
-// sign, other bits (a nonzero difference) and a finite abs_diff.  Such a "lean"
-// pair has no finite-pattern or NaN outputs; its ULP distance is the distance
-// of its codes.  Its ULP bucket goes to copy lane % kRep of the wave's
-// replicated counters `rep` (no ballots, and at most four increments of one
-// element step meet at an address); its abs key, fp64 sums and captures are
-// taken in registers.
+// ------------------------------------------------------------ dense items
+// An item in which many pairs differ (fp32 results that differ by rounding
+// noise everywhere, 16-bit results that round elsewhere), for the isclose test
+// of fp32, bf16 and fp16: every lane finishes its own stage slots in order,
+// the bit-identical pairs among them, so neither phase A's classification nor
+// the queue is needed.  Only the outputs that every pair has are taken per
+// element: the fp64 products, the ULP bucket, the running largest abs_diff
+// (and, in a capture segment, the captured values).  Everything else is
+// settled per vector or per item:
 //
-// Two conservative single-compare tests keep the division off the common path:
-// * tolerance: abs_diff <= fma(|gen|, rtol_lo, atol_lo) with both tolerances
+// * tolerance: abs_diff < fma(|gen|, rtol_lo, atol_lo) with both tolerances
 //   lowered by 2^-21 (lean_tol), which never exceeds the exact allowed bound
-//   fl(atol + fl(rtol * |gen|)): such a pair is close;
-// * rel bound: abs_diff < fl(thr * |ref|), never above fl(thr * den): such a
-//   pair cannot be the rel argmax.
-// A pair that fails either takes slow_elem's exact tests in place (the
-// mismatch counters, the rel argmax).  The capture of rel_diff is settled by
-// fl(cap_rel_lo * |ref|) below and fma(cap_rel_hi, |ref|, cap_rel_hic) above
-// (set_thresholds); the division is left to the thin band between.
+//   fl(atol + fl(rtol * |gen|)): such a pair is close (an infinite abs_diff fails);
+// * rel argmax: best * |ref| >= abs_diff, best the wave's largest rel_diff so
+//   far: such a pair's rel_diff is at most that of an earlier pair;
+// * a pair that fails either test (NaN and Inf do) marks its vector (ballots in
+//   scalar registers, one lane flag per vector); the failing pairs of the
+//   marked vectors go to the queue and slow_elem's exact tests afterwards;
+// * the largest abs_diff is located (lowest index first) only in an item whose
+//   largest exceeds the wave's largest so far;
+// * the ULP distance is the distance of the codes, which is right for pairs of
+//   one sign; the others (found by one accumulated xor) are moved to their
+//   bucket afterwards.  32-bit codes count their bucket in the replicated LDS
+//   counters; of 16-bit codes, a packed form counts the distances >= 1 and >= 2
+//   in registers, and an item with a distance of 4 or more (rare for results
+//   that differ by rounding) counts its buckets in the LDS counters instead.
 //
-// The other slow pairs (opposite signs, +0 against -0, non-finite values) are
-// returned as a mask for the queue and slow_elem.  The lean pairs of a lane
-// come in ascending index order and precede the item's queued pairs, so a
-// strict key comparison keeps the lowest index of a tie.  The bound only
-// rises, so a pair below it now stays below it.  Only the slots of fully loaded
-// vectors are walked (vec_tail takes a partial one's elements; a bit-identical
-// pair, which phase A finished, has a zero difference and is never lean).
-// Taken when every lane has at least 3/4 of those slots slow.  Otherwise
-// `slow` comes back unchanged.
+// What bounds it: VALU issue and, with three waves per SIMD, its latencies.
+// About 20 instructions per fp32 element (7 of them the fp64 products) and 22
+// per 16-bit element, against the 30 of the earlier in-place fp32 loop and the
+// 100 of phase A, the queue and slow_elem.  Whole verdicts: 8191 x 8191 fp32
+// noise 186 -> 138 us (its loads alone 114), 8192 x 8192 bf16 with half of the
+// pairs one ULP apart under the tolerant policy 315 -> 197 us, the ragged batch
+// of 4,096 pairs 1,365 -> 1,250 us.  With the capture's five tests per element
+// behind a branch, a select per ballot and 0.99999 of the largest rel_diff as
+// the bound (which sends every tie to slow_elem), the first two took 158 and
+// 224 us.
 struct LeanTol {
   float rtol, atol;
 };
@@ -1310,7 +1370,8 @@ struct LeanTol {
 // bound fl(A + fl(X)) is at least (X + A) * (1 - 2^-24) - 2^-150.  For A >=
 // 2^-127 the first is the smaller, and for A = 0 rounding's monotonicity
 // orders them.  Tolerances outside [2^-100, 2^100] (zero aside) or a zero
-// tolerance (plain equality) give bounds below zero: no lean pair.
+// tolerance (plain equality) give bounds below zero: every pair is tested
+// exactly.
 __device__ __forceinline__ LeanTol lean_tol(const SegDesc& d) {
   auto ok = [](float t) { return t == 0.0f || (t >= 0x1p-100f && t <= 0x1p100f); };
   if (d.zero_tol || !ok(d.rtol) || !ok(d.atol)) return LeanTol{-1.0f, -1.0f};
@@ -1324,146 +1385,283 @@ __device__ __forceinline__ uint32_t abs_diff_u32(uint32_t a, uint32_t b) {
   return r;
 }
 
-template <int DT, int MODE>
-__device__ __forceinline__ uint64_t phase_b_lean(const SegDesc& d, uint32_t R0, uint64_t slow, uint32_t full,
-                                                 StageP stage, Acc& acc, KVV_LDS uint32_t* rep, uint32_t* wc) {
-  constexpr int V = VecIO<DT>::V;
-  if constexpr (DT != KVV_F32 || MODE != KVV_MODE_ISCLOSE) {
-    return slow;
+// Row (leading zeros - 17, 15 for 0) of the replicated counters that counts
+// code distance x: bucket 15 (2^14 and more) in row 0, bucket 0 in row 15.
+__device__ __forceinline__ uint32_t rep_row(uint32_t x) {
+  uint32_t lz, r;
+  asm("v_ffbh_u32 %0, %1" : "=v"(lz) : "v"(x));  // -1 for 0
+  asm("v_med3_u32 %0, %1, 17, 32" : "=v"(r) : "v"(lz));
+  return r - 17u;
+}
+
+// m = 2 * m + (this lane's bit of `bits`): appends one element's flag to a
+// lane mask in one instruction.
+__device__ __forceinline__ uint32_t push_flag(uint32_t m, uint64_t bits) {
+  uint32_t r;
+  asm("v_addc_co_u32 %0, vcc, %1, %1, %2" : "=v"(r) : "v"(m), "s"(bits) : "vcc");
+  return r;
+}
+
+// (a ^ b) | c in one instruction.
+__device__ __forceinline__ uint32_t or_xor(uint32_t a, uint32_t b, uint32_t c) {
+  uint32_t r;
+  asm("v_bitop3_b32 %0, %1, %2, %3 bitop3:0xbe" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+  return r;
+}
+
+// The lanes where p holds.  (HIP's __ballot takes an int: a select and a
+// compare more per call.)
+__device__ __forceinline__ uint64_t ballot(bool p) { return __builtin_amdgcn_ballot_w64(p); }
+
+// The types and layouts with a dense path.  (16-bit row layouts keep the queue:
+// with the dense path's code in their kernel, row-layout pairs that mostly agree
+// took 2 to 3 % longer, 72.9 -> 74.9 us for an 8 x 16 x 1024 x 128 fp16 view.)
+template <int DT, int MODE, int KIND>
+struct DenseForm {
+  static constexpr bool on = MODE == KVV_MODE_ISCLOSE && ((KIND == K_CONTIG && (DT == KVV_BF16 || DT == KVV_F16)) ||
+                                                          (KIND != K_SCALAR && DT == KVV_F32));
+};
+
+// The float32 values of a dword's codes.
+template <int DT>
+__device__ __forceinline__ void dword_values(uint32_t w, float* f) {
+  if constexpr (DT == KVV_F32) {
+    f[0] = __uint_as_float(w);
+  } else if constexpr (DT == KVV_BF16) {
+    f[0] = __uint_as_float(w << 16);
+    f[1] = __uint_as_float(w & 0xFFFF0000u);
   } else {
-    // (a lane's slots: those of its fully loaded vectors; the others are vec_tail's)
-    if (__ballot((uint32_t)__popcll(slow) * 4u < 3u * (uint32_t)V * (uint32_t)__popc(full))) return slow;
-    const int lane = lane_id();
-    float thr = acc.rel_thr;
-    if (__ballot(!(thr > -__builtin_inff()))) {
-      // no bound yet (the run's first pairs): the largest finite rel_diff of the
-      // wave's slot-0 pairs gives one.  The pairs that reach it are queued, so
-      // every pair skipped below it has a strictly smaller rel_diff than a
-      // pair slow_elem will see.
-      const float g = stage_elem<float>(stage, lane, 0), r = stage_elem<float>(stage, 64 + lane, 0);
-      const float rel = fabsf(g - r) / (fabsf(r) + 1e-12f);
-      const float m = wave_max_f32((slow & 1u) && __builtin_isfinite(rel) ? rel : -__builtin_inff());
-      if (m > -__builtin_inff()) {
-        const float t = rel_threshold(m);
-        thr = t > thr ? t : thr;
+    f[0] = Elem<DT>::f32((uint16_t)w);
+    f[1] = Elem<DT>::f32((uint16_t)(w >> 16));
+  }
+}
+
+// What phase_dense leaves, per lane in the slow-mask layout: the pairs for
+// slow_elem's exact tests, and (NZ, for near_entries) the differing pairs.
+struct DenseLeft {
+  uint32_t test, differ;
+};
+
+// Finishes an item whose lanes all hold `nu` full vectors (and no partial one).
+// CAP: a batch launch, whose fp32 segments may capture.
+template <int DT, bool NZ, bool CAP>
+__device__ __forceinline__ DenseLeft phase_dense(const SegDesc& d, uint32_t R0, int nu, StageP stage, Acc& acc,
+                                                KVV_LDS uint32_t* rep, uint32_t* wc) {
+  using T = typename Elem<DT>::T;
+  constexpr int V = VecIO<DT>::V;
+  constexpr int W = Elem<DT>::width;
+  constexpr int EPD = 32 / W;  // elements per dword
+  const int lane = lane_id();
+  const LeanTol lt0 = lean_tol(d);
+  const float rt = uniform(lt0.rtol);
+  float at = lt0.atol;
+  asm("" : "+v"(at));  // (in a vector register: an instruction reads one scalar register)
+  // the rel bound: the wave's largest rel_diff so far (a NaN bounds like +inf).
+  // fma(best, |ref|, -abs_diff) >= 0 tells, exactly, that best * |ref| >=
+  // abs_diff, so abs_diff / den rounds to at most best: no argmax, since the
+  // pairs of earlier items keep a tie.  (Below 2^-40 the fma may underflow.)
+  float thr = acc.rel_best != acc.rel_best ? __builtin_inff() : (acc.rel_best > 0x1p-40f ? acc.rel_best : -__builtin_inff());
+  if (!(thr > 0.0f)) {
+    // no bound yet (the run's first pairs): 0.99999 of the largest finite
+    // rel_diff of the wave's first pairs, so that the pairs that reach it are
+    // tested and every pair skipped has a strictly smaller rel_diff
+    float g[2], r[2];
+    dword_values<DT>(stage_vec(stage, lane).x, g);
+    dword_values<DT>(stage_vec(stage, 64 + lane).x, r);
+    const float rel = fabsf(g[0] - r[0]) / (fabsf(r[0]) + 1e-12f);
+    const float t = rel_threshold(wave_max(__builtin_isfinite(rel) ? rel : 0.0f));
+    if (t > 0x1p-40f) thr = t;
+  }
+  thr = uniform(thr);
+  float im = -1.0f;  // the lane's largest abs_diff of the item (NaN aside), and its first vector that holds it
+  int iu = 0;
+  uint32_t fv = 0;  // the lane's vectors with a failing pair (vector u at bit nu - 1 - u)
+  uint32_t sx = 0, dm = 0, c1 = 0, c2 = 0, differ = 0;
+  const bool capseg = CAP && DT == KVV_F32 && (d.flags & kFlagCaptureElems) != 0;
+  uint32_t cma = 0, cmr = 0, nzc = 0;
+  const uint32_t ca0 = uniform(d.cap_key[0]) & 0x7FFFFFFFu;
+  const float crlo = uniform(d.cap_rel_lo);
+#pragma unroll 1
+  for (int u = 0; u < nu; ++u) {
+    const uint4 gq = stage_vec(stage, (2 * u) * 64 + lane);
+    const uint4 rq = stage_vec(stage, (2 * u + 1) * 64 + lane);
+    const uint32_t gw[4] = {gq.x, gq.y, gq.z, gq.w};
+    const uint32_t rw[4] = {rq.x, rq.y, rq.z, rq.w};
+    uint64_t fail = 0;
+    const float im0 = im;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      sx = or_xor(gw[j], rw[j], sx);
+      if constexpr (W == 32) {
+        atomicAdd((uint32_t*)(rep + rep_row(abs_diff_u32(gw[j], rw[j])) * kRep + (lane & (kRep - 1))), 1u);
+      } else {
+        const u16x2 gh = __builtin_bit_cast(u16x2, gw[j]), rh = __builtin_bit_cast(u16x2, rw[j]);
+        const u16x2 dist = __builtin_elementwise_max(gh, rh) - __builtin_elementwise_min(gh, rh);
+        const uint32_t dw = __builtin_bit_cast(uint32_t, dist);
+        const uint32_t one = pk_nonzero16(dw);
+        dm |= dw;
+        c1 += one;  // (at most 16 per half and item: the halves never carry)
+        c2 += (dw >> 1) & 0x7FFF7FFFu;  // distances below 4: 1 for 2 and 3 (else this count is not used)
+        if constexpr (NZ) differ |= one << (u * 4 + j);
       }
-    }
-    const LeanTol lt = lean_tol(d);
-    const bool zt = d.zero_tol != 0;
-    // the ULP counters by leading zeros of the distance: row j - 17 for bucket
-    // 32 - j, bucket 15 (distances of 2^14 and more) in row 0
-    KVV_LDS uint32_t* const mine = rep + (lane & (kRep - 1)) - 17 * kRep;
-    // the lane's largest lean abs_diff (its bits; abs_diff >= 0) and its slot
-    uint32_t best = acc.gabs_k > kZeroKey ? acc.gabs_k & 0x7FFFFFFFu : 0u;
-    int bslot = -1;
-    uint32_t leanm = 0;
-    const bool capseg = (d.flags & kFlagCaptureElems) != 0;
-    uint32_t cm[2] = {0u, 0u};  // capture segment: the lean slots whose abs / rel value is captured
-    // (the thresholds in registers: loads of them inside the loop would wait on its LDS atomics)
-    const uint32_t ca0 = uniform(d.cap_key[0]) & 0x7FFFFFFFu, ck1 = uniform(d.cap_key[1]);
-    const float crlo = __uint_as_float(uniform(__float_as_uint(d.cap_rel_lo)));
-    const float crhi = __uint_as_float(uniform(__float_as_uint(d.cap_rel_hi)));
-    const float crhc = __uint_as_float(uniform(__float_as_uint(d.cap_rel_hic)));
+      float g[2], r[2];
+      dword_values<DT>(gw[j], g);
+      dword_values<DT>(rw[j], r);
 #pragma unroll
-    for (int u = 0; u < kUnroll; ++u) {
-      if (__ballot(((slow >> (u * V)) & 0xFu) != 0) == 0) continue;
-      const uint4 gq = stage_vec(stage, (2 * u) * 64 + lane);
-      const uint4 rq = stage_vec(stage, (2 * u + 1) * 64 + lane);
-      const uint32_t gw[4] = {gq.x, gq.y, gq.z, gq.w};
-      const uint32_t rw[4] = {rq.x, rq.y, rq.z, rq.w};
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int p = u * 4 + e;
-        const float g = __uint_as_float(gw[e]), r = __uint_as_float(rw[e]);
-        const float ad = fabsf(g - r);
-        const uint32_t ab = __float_as_uint(ad);
-        // (a loaded vector; one sign and other bits: a nonzero difference)
-        const bool lean = ((full >> u) & 1u) && (int32_t)(gw[e] ^ rw[e]) > 0 && ad < __builtin_inff();
-        leanm |= (lean ? 1u : 0u) << p;
-        if (lean) {
-          const bool tol = ad <= fmaf(fabsf(g), lt.rtol, lt.atol);
-          const bool below = ad < thr * fabsf(r);
-          if (!(tol && below)) {
-            // a mismatch or a rel-argmax candidate (slow_elem's tests, exactly)
-            const float rel = ad / (fabsf(r) + 1e-12f);
-            const uint32_t rk = fkey(rel);
-            const uint32_t idx = R0 + (uint32_t)((u * 64 + lane) * V + e);
-            if (!tol && (zt || !(ad <= d.atol + fabsf(d.rtol * g)))) {
-              ++acc.nmm;
-              acc.first_mm = idx < acc.first_mm ? idx : acc.first_mm;
-              acc.mm_abs = fkey(ad) > acc.mm_abs ? fkey(ad) : acc.mm_abs;
-              acc.mm_rel = rk > acc.mm_rel ? rk : acc.mm_rel;
-            }
-            if (!below && better32(rk, idx, acc.grel_k, acc.grel_i)) {
-              acc.grel_k = rk;
-              acc.grel_i = idx;
-              const float t = rel_threshold(rel);
-              thr = t > thr ? t : thr;
-            }
-          }
-          if (ab > best) {
-            best = ab;
-            bslot = p;
-          }
-          // one sign: the ULP distance is the distance of the codes (nonzero here)
-          const uint32_t lz = (uint32_t)__builtin_clz(abs_diff_u32(gw[e], rw[e]));
-          atomicAdd((uint32_t*)(mine + (lz > 17u ? lz : 17u) * kRep), 1u);
-          const double g64 = (double)g, r64 = (double)r;
-          const double d64 = g64 - r64;
-          acc.s[0] = fma(g64, g64, acc.s[0]);
-          acc.s[1] = fma(r64, r64, acc.s[1]);
-          acc.s[2] = fma(g64, r64, acc.s[2]);
-          acc.s[3] = fma(d64, d64, acc.s[3]);
+      for (int e = 0; e < EPD; ++e) {
+        const float ad = fabsf(g[e] - r[e]);
+        const bool ok = (ad < fmaf(fabsf(g[e]), rt, at)) & (fmaf(thr, fabsf(r[e]), -ad) >= 0.0f);
+        fail |= ballot(!ok);
+        im = fmaxf(im, ad);
+        const double g64 = (double)g[e], r64 = (double)r[e];
+        const double d64 = g64 - r64;
+        acc.s[0] = fma(g64, g64, acc.s[0]);
+        acc.s[1] = fma(r64, r64, acc.s[1]);
+        acc.s[2] = fma(g64, r64, acc.s[2]);
+        acc.s[3] = fma(d64, d64, acc.s[3]);
+        if constexpr (DT == KVV_F32 && CAP) {
           if (capseg) {
-            const bool hi = ad >= fmaf(crhi, fabsf(r), crhc);
-            cm[0] |= (ab >= ca0 ? 1u : 0u) << p;
-            cm[1] |= (hi ? 1u : 0u) << p;
-            if (!hi && !(ad < crlo * fabsf(r)) && fkey(ad / (fabsf(r) + 1e-12f)) >= ck1) cm[1] |= 1u << p;
+            // captured: abs_diff at its threshold, rel_diff at (or a rounding below) its own; the zeros are not
+            const uint64_t nz = ballot(!(ad == 0.0f));
+            nzc += (uint32_t)__popcll(nz);
+            cma = push_flag(cma, ballot(__float_as_uint(ad) >= ca0));
+            cmr = push_flag(cmr, ballot(!(ad < crlo * fabsf(r[e]))) & nz);
           }
         }
       }
     }
-    acc.rel_thr = thr;
-    if (bslot >= 0) {
-      acc.gabs_k = best | kZeroKey;
-      acc.gabs_i = R0 + (uint32_t)((((bslot >> 2) * 64 + lane) * V) + (bslot & 3));
+    fv = push_flag(fv, fail);
+    iu = im > im0 ? u : iu;
+  }
+  if constexpr (W == 16) {
+    const uint32_t ge1 = (c1 & 0xFFFFu) + (c1 >> 16);
+    acc.nfast += (uint32_t)(nu * V) - ge1;
+    if (__ballot((dm & 0xFFFCFFFCu) != 0)) {
+      // a distance of 4 or more: the buckets of the item's differing pairs one by one
+#pragma unroll 1
+      for (int u = 0; u < nu; ++u) {
+        const uint4 gq = stage_vec(stage, (2 * u) * 64 + lane);
+        const uint4 rq = stage_vec(stage, (2 * u + 1) * 64 + lane);
+        const uint32_t gw[4] = {gq.x, gq.y, gq.z, gq.w};
+        const uint32_t rw[4] = {rq.x, rq.y, rq.z, rq.w};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const uint32_t lo = abs_diff_u32(gw[j] & 0xFFFFu, rw[j] & 0xFFFFu), hi = abs_diff_u32(gw[j] >> 16, rw[j] >> 16);
+          if (lo) atomicAdd((uint32_t*)(rep + rep_row(lo) * kRep + (lane & (kRep - 1))), 1u);
+          if (hi) atomicAdd((uint32_t*)(rep + rep_row(hi) * kRep + (lane & (kRep - 1))), 1u);
+        }
+      }
+    } else {
+      const uint32_t ge2 = (c2 & 0xFFFFu) + (c2 >> 16);
+      atomicAdd((uint32_t*)(rep + rep_at(1)), ge1 - ge2);
+      atomicAdd((uint32_t*)(rep + rep_at(2)), ge2);
     }
-    const uint64_t rare = slow & ~(uint64_t)leanm;
+  }
+  // pairs of opposite signs: from the bucket of their codes' distance to their own
+  constexpr uint32_t kSigns = W == 32 ? 0x80000000u : 0x80008000u;
+  if (__ballot((sx & kSigns) != 0)) {
+#pragma unroll 1
+    for (int p = 0; p < nu * V; ++p) {
+      const int u = p / V, e = p % V;
+      const T gc = stage_elem<T>(stage, (2 * u) * 64 + lane, e), rc = stage_elem<T>(stage, (2 * u + 1) * 64 + lane, e);
+      if (Elem<DT>::sign(gc) != Elem<DT>::sign(rc)) {
+        atomicAdd((uint32_t*)(rep + rep_row(abs_diff_u32(gc, rc)) * kRep + (lane & (kRep - 1))), ~0u);
+        atomicAdd((uint32_t*)(rep + rep_at(pair_bucket<DT>(gc, rc))), 1u);
+      }
+    }
+  }
+  // the item's largest abs_diff, where it exceeds the wave's so far: its lowest
+  // index is in the first vector (vectors, then lanes) that holds it
+  if (__ballot(im > acc.abs_best)) {
+    const float top = wave_max(im);
+    const uint32_t v = wave_min(im == top ? (uint32_t)(iu * 64 + lane) : kNone32);
+    const int u = (int)(v >> 6), l = (int)(v & 63u), e = lane & (V - 1);
+    const float ad = fabsf(Elem<DT>::f32(stage_elem<T>(stage, (2 * u) * 64 + l, e)) -
+                           Elem<DT>::f32(stage_elem<T>(stage, (2 * u + 1) * 64 + l, e)));
+    const int first = __ffsll((long long)__ballot(ad == top)) - 1;  // (below V)
+    const uint32_t idx = R0 + v * V + (uint32_t)first, key = __float_as_uint(top) | kZeroKey;
+    if (lane == 0 && better32(key, idx, acc.gabs_k, acc.gabs_i)) {
+      acc.gabs_k = key;
+      acc.gabs_i = idx;
+    }
+    acc.abs_best = uniform(top);
+  }
+  if constexpr (NZ) {
+    // near-zero pairs with a large abs_diff (none unless the item's largest is one)
+    if (__ballot(im > d.nz_bad)) {
+#pragma unroll 1
+      for (int p = 0; p < nu * V; ++p) {
+        const int u = p / V, e = p % V;
+        const T gc = stage_elem<T>(stage, (2 * u) * 64 + lane, e), rc = stage_elem<T>(stage, (2 * u + 1) * 64 + lane, e);
+        const float r = Elem<DT>::f32(rc);
+        wave_add(wc, LC_NEARBAD, fabsf(r) <= d.nz_abs && fabsf(Elem<DT>::f32(gc) - r) > d.nz_bad);
+      }
+    }
+  }
+  // the failing pairs (slow-mask layout), for slow_elem's exact tests
+  uint32_t left = 0;
+  if (__ballot(fv != 0)) {
+#pragma unroll 1
+    for (int u = 0; u < nu; ++u) {
+      const bool marked = (fv >> (nu - 1 - u)) & 1u;
+      if (__ballot(marked) == 0) continue;
+      auto test = [&](uint32_t gd, uint32_t rd, int j) {
+        float g[2], r[2];
+        dword_values<DT>(gd, g);
+        dword_values<DT>(rd, r);
+#pragma unroll
+        for (int e = 0; e < EPD; ++e) {
+          const float ad = fabsf(g[e] - r[e]);
+          const bool ok = (ad < fmaf(fabsf(g[e]), rt, at)) & (fmaf(thr, fabsf(r[e]), -ad) >= 0.0f);
+          left |= (ok ? 0u : 1u) << (e * 16 + u * 4 + j);
+        }
+      };
+      if constexpr (W == 32) {
+        const uint4 gq = stage_vec(stage, (2 * u) * 64 + lane), rq = stage_vec(stage, (2 * u + 1) * 64 + lane);
+        test(gq.x, rq.x, 0);
+        test(gq.y, rq.y, 1);
+        test(gq.z, rq.z, 2);
+        test(gq.w, rq.w, 3);
+      } else {
+        // (a dword at a time: the vector form took 27 registers more)
+#pragma unroll 1
+        for (int j = 0; j < 4; ++j)
+          test(stage_elem<uint32_t>(stage, (2 * u) * 64 + lane, j), stage_elem<uint32_t>(stage, (2 * u + 1) * 64 + lane, j), j);
+      }
+    }
+  }
+  if constexpr (DT == KVV_F32 && CAP) {
     if (capseg) {
-      // the captured values of the lean pairs, lane by lane in slot order, from
-      // the stage, after the run's captures so far; the lean pairs not captured
-      // are nonzero values below the threshold
-      const uint32_t nl = (uint32_t)__popc(leanm);
-      const uint32_t c0 = (uint32_t)__popc(cm[0]), c1 = (uint32_t)__popc(cm[1]);
-      const uint32_t pk = c0 | (c1 << 16);  // (a wave adds at most 1024 to each half)
+      // the captured values, lane by lane, from the stage, after the run's
+      // captures so far (element k of the lane sits at bit nu * V - 1 - k);
+      // the nonzero values not captured are below the threshold
+      const uint32_t na = (uint32_t)__popc(cma), nr = (uint32_t)__popc(cmr);
+      const uint32_t pk = na | (nr << 16);  // (a wave adds at most 1024 to each half)
       const uint32_t incl = wave_incl_scan(pk);
       const uint32_t tot = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
-      const uint32_t nb = wave_sum((nl - c0) | ((nl - c1) << 16));
-      if (tot | nb) {
-        const uint32_t base = wc[WC_CBASE], f0 = wc[WC_CFILL], f1 = wc[WC_CFILL + 1];
-        const uint32_t ex = incl - pk;
-        float* pa = d.cap_buf[0] + base + f0 + (ex & 0xFFFFu);
-        float* pr = d.cap_buf[1] + base + f1 + (ex >> 16);
+      const uint32_t base = wc[WC_CBASE], q0 = wc[WC_CFILL], q1 = wc[WC_CFILL + 1];
+      const uint32_t ex = incl - pk;
+      float* pa = d.cap_buf[0] + base + q0 + (ex & 0xFFFFu);
+      float* pr = d.cap_buf[1] + base + q1 + (ex >> 16);
 #pragma unroll
-        for (int x = 0; x < 2; ++x) {
-          for (uint32_t mk = cm[x]; mk; mk &= mk - 1) {
-            const int p = __builtin_ctz(mk), u = p >> 2, e = p & 3;
-            const float g = stage_elem<float>(stage, (2 * u) * 64 + lane, e);
-            const float r = stage_elem<float>(stage, (2 * u + 1) * 64 + lane, e);
-            const float ad = fabsf(g - r);
-            if (x == 0) *pa++ = ad; else *pr++ = ad / (fabsf(r) + 1e-12f);
-          }
-        }
-        if (lane == 0) {
-          wc[WC_CFILL] = f0 + (tot & 0xFFFFu);
-          wc[WC_CFILL + 1] = f1 + (tot >> 16);
-          wc[WC_BELOW] += nb & 0xFFFFu;
-          wc[WC_BELOW + 1] += nb >> 16;
+      for (int x = 0; x < 2; ++x) {
+        for (uint32_t mk = x == 0 ? cma : cmr; mk; mk &= mk - 1) {
+          const int p = nu * V - 1 - __builtin_ctz(mk), u = p >> 2, e = p & 3;
+          const float g = stage_elem<float>(stage, (2 * u) * 64 + lane, e);
+          const float r = stage_elem<float>(stage, (2 * u + 1) * 64 + lane, e);
+          const float ad = fabsf(g - r);
+          if (x == 0) *pa++ = ad; else *pr++ = ad / (fabsf(r) + 1e-12f);
         }
       }
+      if (lane == 0) {
+        wc[WC_CFILL] = q0 + (tot & 0xFFFFu);
+        wc[WC_CFILL + 1] = q1 + (tot >> 16);
+        wc[WC_BELOW] += nzc - (tot & 0xFFFFu);
+        wc[WC_BELOW + 1] += nzc - (tot >> 16);
+      }
     }
-    return rare;
   }
+  return DenseLeft{left, differ};
 }
 
 // Adds the wave's replicated ULP-bucket counters into its LDS counters and
@@ -1473,8 +1671,8 @@ __device__ __forceinline__ void fold_rep(KVV_LDS uint32_t* rep, uint32_t* wc) {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  // row i counts bucket 15 - i (phase_b_lean)
-  if (lane < kBuckets - 1) {
+  // (row i counts bucket 15 - i; a pair taken back leaves its copy's count modulo 2^32)
+  if (lane < kBuckets) {
     uint32_t t = 0;
 #pragma unroll
     for (int c = 0; c < kRep; ++c) {
@@ -2082,6 +2280,12 @@ __device__ inline void fold_block_record(const LdsRecord* rec, const RunCols& ou
   }
 }
 
+// When the dense path takes an item over from phase A and the queue: a dense
+// item costs about as much as 7 (16-bit) or 3 (fp32) queue steps of 64 slow
+// pairs, i.e. a quarter of the item's.  The kDenseRun items after it skip phase A.
+constexpr uint32_t kDenseShare = 4;
+constexpr int kDenseRun = 15;
+
 // ------------------------------------------------------------ scan kernel
 // LDS of one scan block: per wave, its item's vectors (SW uint4: kUnroll
 // vectors of each tensor per lane), its queue of stage positions (NQ entries:
@@ -2105,8 +2309,9 @@ struct ScanLds {
   static constexpr bool vec = KIND != K_SCALAR;
   using QG = QueueGeom<DT>;
   // (the scalar kind stages nothing, but its waves leave their run records there)
+  static constexpr bool rep = vec && (KIND == K_CONTIG || DT == KVV_F32);
   using type = ScanShared<vec ? 2 * kUnroll * 64 : (kColU32 * 4 + kColU64 * 8 + 15) / 16, vec ? 64 * QG::slots : 2,
-                          vec ? QG::rep_words : 1, SampleWords<DT>::words>;
+                          rep ? QG::rep_words : 1, SampleWords<DT>::words>;
 };
 
 // Per-item near-zero count of the wave (feeds the compacted-rank prefix of near_kernel).
@@ -2120,11 +2325,10 @@ __device__ __forceinline__ void near_item_count(const ScanArgs& a, int64_t item,
 }
 
 // Phase A variant by wave-uniform conditions (near-zero counting; the quick or
-// careful dot form), then the lowest bit-identical index while it can still be
-// an argmax.  `careful` counts the items left in the careful form.
+// careful dot form).  `careful` counts the items left in the careful form.
 template <int DT>
-__device__ __forceinline__ uint64_t phase_a_any(const SegDesc& d, int64_t L0, uint32_t R0, StageP stage,
-                                                uint32_t full, Acc& acc, uint32_t& careful) {
+__device__ __forceinline__ PhaseA phase_a_any(const SegDesc& d, StageP stage, uint32_t full, uint32_t& careful) {
+  PhaseA o;
   if (!d.fast) {
     // no element can take the fast path: all elements of the full vectors are slow
     uint64_t all = 0;
@@ -2133,11 +2337,11 @@ __device__ __forceinline__ uint64_t phase_a_any(const SegDesc& d, int64_t L0, ui
       slot_of<Elem<DT>::width>(p, u, e);
       if ((full >> u) & 1u) all |= 1ull << p;
     }
-    return all;
+    o.slow = all;
+    o.nfast = o.nnear = 0;
+    o.esq = 0.0;
+    return o;
   }
-  const bool track =
-      __ballot(acc.first_fast == kNone32 && (acc.gabs_k <= 0x80000000u || acc.grel_k <= 0x80000000u)) != 0;
-  PhaseA o;
   if (d.flags & KVV_FLAG_NEAR_ZERO) {
     o = phase_a<DT, true>(d, stage, full);
   } else if constexpr (DotForm<DT>::on) {
@@ -2158,12 +2362,19 @@ __device__ __forceinline__ uint64_t phase_a_any(const SegDesc& d, int64_t L0, ui
   } else {
     o = phase_a<DT, false>(d, stage, full);
   }
+  return o;
+}
+
+// Joins what phase A settled to the accumulators.
+template <int DT>
+__device__ __forceinline__ void phase_a_join(const SegDesc& d, const PhaseA& o, uint32_t R0, uint32_t full, Acc& acc) {
+  if (!d.fast) return;
+  const bool track =
+      __ballot(acc.first_fast == kNone32 && (acc.gabs_k <= 0x80000000u || acc.grel_k <= 0x80000000u)) != 0;
   acc.e_sq += o.esq;
   acc.nfast += o.nfast;
   acc.nnear_fast += o.nnear;
-  const uint64_t slow = o.slow;
-  if (track) track_first_fast<DT>(R0, full, slow, acc);
-  return slow;
+  if (track) track_first_fast<DT>(R0, full, o.slow, acc);
 }
 
 // A wave of a single-segment launch leaves its run record in its own stage
@@ -2202,7 +2413,7 @@ __device__ inline void block_record_part(const ScanArgs& a, SM& sm, Acc& acc, ui
 // NZ: a single fp16/bf16 pair whose near-zero diagnostics are taken as entries
 // (kFlagNearEntries); the vector kinds with the dtype's isclose test only.
 template <int DT, int MODE, int KIND, bool BATCH, bool NZ = false>
-__global__ __launch_bounds__(kBlock, BATCH ? 3 : 1) void scan_kernel(ScanArgs a) {
+__global__ __launch_bounds__(kBlock, BATCH || NZ ? 3 : 1) void scan_kernel(ScanArgs a) {
   static_assert(!NZ || (!BATCH && KIND != K_SCALAR && MODE == KVV_MODE_ISCLOSE && Elem<DT>::width == 16 &&
                         Elem<DT>::is_float), "near-zero entries: single fp16/bf16 pairs, vector kinds");
   __shared__ typename ScanLds<DT, KIND>::type sm;
@@ -2212,12 +2423,10 @@ __global__ __launch_bounds__(kBlock, BATCH ? 3 : 1) void scan_kernel(ScanArgs a)
   const int tid = threadIdx.x, w = (int)uniform((uint32_t)(tid >> 6)), lane = tid & 63;
   uint32_t* wc = sm.wcnt[w];
   if (lane < WC_COUNT) wc[lane] = 0;
-  // the dense path's replicated ULP-bucket counters (fp32 isclose, vector kinds)
-  constexpr bool kLean = DT == KVV_F32 && MODE == KVV_MODE_ISCLOSE && KIND != K_SCALAR;
+  // the dense path's replicated ULP-bucket counters
+  constexpr bool kDense = DenseForm<DT, MODE, KIND>::on;
   KVV_LDS uint32_t* const rep = (KVV_LDS uint32_t*)sm.rep[w];
-  if constexpr (kLean) {
-    for (int i = lane; i < kBuckets * kRep; i += 64) rep[i] = 0;
-  }
+  bool rep_used = false;  // (cleared at the wave's first dense item)
   if constexpr (!BATCH) {
     if (tid == 0) sm.done = 0;
   }
@@ -2329,22 +2538,33 @@ __global__ __launch_bounds__(kBlock, BATCH ? 3 : 1) void scan_kernel(ScanArgs a)
       const int64_t L1 = base + d.item_elems < d.n ? base + d.item_elems : d.n;
       full = load_item<DT, KIND>(d, base, L1, gv, rv, rcur, rmap);
     }
-    for (; it < run_end; ++it) {
-      const int64_t L0 = (it - d.item_begin) * (int64_t)d.item_elems;
-      const int64_t L1 = L0 + d.item_elems < d.n ? L0 + d.item_elems : d.n;
-      const uint32_t R0 = (uint32_t)(L0 - base);
-      if constexpr (KIND == K_SCALAR) {
+    if constexpr (KIND == K_SCALAR) {
+      for (; it < run_end; ++it) {
+        const int64_t L0 = (it - d.item_begin) * (int64_t)d.item_elems;
+        const int64_t L1 = L0 + d.item_elems < d.n ? L0 + d.item_elems : d.n;
         scan_item_scalar<DT, MODE>(d, L0, L1, base, acc, wc);
         sample_range<DT, MODE>(d, L0, L1, acc, a.sample_abs, a.sample_rel);
-      } else {
+        if (d.flags & KVV_FLAG_NEAR_ZERO) near_item_count(a, it, acc, wc, near_prev);
+      }
+    } else {
+      constexpr int QS = QueueGeom<DT>::slots;
+      StageP stage = (StageP)sm.stage[w];
+      // the current item: its elements [L0, L1), R0 = L0 from the run's first, the lanes' full vectors
+      int64_t L0 = base, L1 = base;
+      uint32_t R0 = 0, full_now = 0;
+      NearItem ni{};
+      // item `it`: staged, the next item's loads issued, its samples and near-zero masks taken
+      auto open_item = [&]() {
+        L0 = (it - d.item_begin) * (int64_t)d.item_elems;
+        L1 = L0 + d.item_elems < d.n ? L0 + d.item_elems : d.n;
+        R0 = (uint32_t)(L0 - base);
         if (full != (1u << kUnroll) - 1) patch_partial<DT, KIND>(d, L0, L1, full, gv, rv);
 #pragma unroll
         for (int u = 0; u < kUnroll; ++u) {
           sm.stage[w][(2 * u) * 64 + lane] = gv[u];
           sm.stage[w][(2 * u + 1) * 64 + lane] = rv[u];
         }
-        const uint32_t full_now = full;
-        StageP stage = (StageP)sm.stage[w];
+        full_now = full;
         // the next item of the run: its loads fly while this one finishes
         if (it + 1 < run_end) {
           const int64_t N1 = L1 + d.item_elems < d.n ? L1 + d.item_elems : d.n;
@@ -2353,30 +2573,9 @@ __global__ __launch_bounds__(kBlock, BATCH ? 3 : 1) void scan_kernel(ScanArgs a)
         // (an input-select segment's samples and sampled sums come from the input-select kernels)
         if (!dense && !(d.flags & kFlagInputSelect))
           sample_item<DT, MODE>(d, L0, L1, stage, acc, a.sample_abs, a.sample_rel, cur, sb, ba, br, mh);
-        NearItem ni{};
         if constexpr (NZ) ni = near_item<DT>(d, stage, L0, L1, full_now);
-        const uint64_t slow = phase_a_any<DT>(d, L0, R0, stage, full_now, acc, careful);
-        if constexpr (NZ) near_entries<DT>(ni, slow, full_now, stage, sink);
-        // what is left for the queue after an in-place pass over an item of mostly slow pairs
-        uint64_t left = slow;
-        if (__ballot(slow != 0)) {
-          if (kLean && !(d.flags & kFlagNearAny)) left = phase_b_lean<DT, MODE>(d, R0, slow, full_now, stage, acc, rep, wc);
-          else if (phase_b_dense<DT, MODE>(d, R0, slow, stage, acc, wc)) left = 0;
-        }
-        if (__ballot(left != 0)) {
-          constexpr int QS = QueueGeom<DT>::slots;
-          uint32_t nq = queue_all<QS>(left, sm.queue[w]);
-          // more than the queue holds: QS slots of every lane at a time
-          const bool split = nq > 64u * QS;
-#pragma unroll 1
-          for (int p0 = 0;; p0 += QS) {
-            if (split) nq = queue_part<QS>((uint32_t)(left >> p0), p0, sm.queue[w]);
-            if (nq) phase_b<DT, MODE>(d, R0, nq, stage, sm.queue[w], acc, wc);
-            if (!split || p0 + QS >= VecIO<DT>::NE) break;
-          }
-        }
-        // (every lane enters: slow_elem's wave-wide steps then see the whole wave)
-        if (__ballot(full_now != (1u << kUnroll) - 1)) vec_tail<DT, MODE>(d, L0, L1, R0, full_now, stage, acc, wc);
+      };
+      auto close_item = [&]() {
         if constexpr (NZ) {
           // every near-zero element of the item joins the run's count
           if (lane == 0) acc.nnear_fast += ni.total;
@@ -2384,12 +2583,87 @@ __global__ __launch_bounds__(kBlock, BATCH ? 3 : 1) void scan_kernel(ScanArgs a)
         }
         if (dense && !(d.flags & kFlagInputSelect))
           dense_samples<DT, MODE>(d, L0, L1, stage, acc, a.sample_abs, a.sample_rel, mh);
+        if (d.flags & KVV_FLAG_NEAR_ZERO) near_item_count(a, it, acc, wc, near_prev);
+      };
+      // the queue: what it holds, then (more than that) QS slots of every lane at a time
+      auto drain = [&](uint64_t left, uint32_t count, auto&& run) {
+        const bool split = count > 64u * QS;
+#pragma unroll 1
+        for (int p0 = 0;; p0 += QS) {
+          if (split) count = queue_part<QS>((uint32_t)(left >> p0), p0, sm.queue[w]);
+          if (count) run(count);
+          if (!split || p0 + QS >= VecIO<DT>::NE) break;
+        }
+      };
+      // whether lanes with the full vectors `f` and elements [e0, e1) make a dense item: nu whole vectors each
+      int nu = 0;
+      auto dense_fits = [&](uint32_t f, int64_t e0, int64_t e1) {
+        const uint32_t fu = uniform(f);
+        nu = __popc(fu);
+        // (16-bit capture segments keep the queue: the captures of phase_dense are fp32's)
+        constexpr uint32_t kOther = KVV_FLAG_NEAR_ZERO | (DT == KVV_F32 ? 0u : kFlagCaptureElems);
+        return d.fast && !(d.flags & kOther) && fu == (1u << nu) - 1u && nu > 0 && __ballot(f != fu) == 0 &&
+               e1 - e0 == (int64_t)nu * 64 * VecIO<DT>::V;
+      };
+      while (it < run_end) {
+        // items by phase A and the queue, until one (opened) has at least
+        // 1/kDenseShare of its pairs slow
+        bool many = false;
+        for (; it < run_end; ++it) {
+          open_item();
+          const PhaseA pa = phase_a_any<DT>(d, stage, full_now, careful);
+          const uint64_t slow = pa.slow;
+          uint32_t nq = 0;
+          if (__ballot(slow != 0)) {
+            nq = queue_all<QS>(slow, sm.queue[w]);
+            if constexpr (kDense) {
+              // (first against the least such item, a constant)
+              if (__builtin_expect(nq * kDenseShare >= 64u * VecIO<DT>::V, 0) && dense_fits(full_now, L0, L1) &&
+                  nq * kDenseShare >= (uint32_t)nu * 64u * VecIO<DT>::V) {
+                many = true;
+                break;
+              }
+            }
+          }
+          phase_a_join<DT>(d, pa, R0, full_now, acc);
+          if constexpr (NZ) near_entries<DT>(ni, slow, full_now, stage, sink);
+          // (32- and 64-bit types without a dense path)
+          if constexpr (!kDense) {
+            if (nq && phase_b_dense<DT, MODE>(d, R0, slow, stage, acc, wc)) nq = 0;
+          }
+          if (nq) drain(slow, nq, [&](uint32_t count) { phase_b<DT, MODE>(d, R0, count, stage, sm.queue[w], acc, wc); });
+          // (every lane enters: slow_elem's wave-wide steps then see the whole wave)
+          if (__ballot(full_now != (1u << kUnroll) - 1)) vec_tail<DT, MODE>(d, L0, L1, R0, full_now, stage, acc, wc);
+          close_item();
+        }
+        if constexpr (kDense) {
+          // dense items: the opened one and up to kDenseRun after it, without phase A.  (A loop of its own, with
+          // a phase B of its own: in one loop, the common path of mostly identical pairs was 2 to 6 % slower.)
+          if (many && !rep_used) {
+            for (int i = lane; i < kBuckets * kRep; i += 64) rep[i] = 0;
+            __builtin_amdgcn_wave_barrier();
+            rep_used = true;
+          }
+          for (int k = 0; many; ++k) {
+            const DenseLeft o = phase_dense<DT, NZ, BATCH>(d, R0, nu, stage, acc, rep, wc);
+            if constexpr (NZ) near_entries<DT>(ni, o.differ, full_now, stage, sink);
+            if (__ballot(o.test != 0)) {
+              drain(o.test, queue_all<QS>((uint64_t)o.test, sm.queue[w]), [&](uint32_t count) {
+                phase_b<DT, MODE, true>(d, R0, count, stage, sm.queue[w], acc, wc, rep);
+              });
+            }
+            close_item();
+            ++it;
+            many = k < kDenseRun && it < run_end &&
+                   dense_fits(full, L1, L1 + d.item_elems < d.n ? L1 + d.item_elems : d.n);
+            if (many) open_item();
+          }
+        }
       }
-      if (d.flags & KVV_FLAG_NEAR_ZERO) near_item_count(a, it, acc, wc, near_prev);
     }
     // the run's buffered samples join its record
     if constexpr (KIND != K_SCALAR) sbuf_store<DT, MODE>(d, sb, ba, br, a.sample_abs, a.sample_rel, acc, mh);
-    if constexpr (kLean) fold_rep(rep, wc);
+    if (kDense && rep_used) fold_rep(rep, wc);
     if (BATCH && (d.flags & kFlagCaptureElems)) {
       // the run's record (its first element and captured counts) and its values below the thresholds
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");

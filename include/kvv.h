@@ -160,7 +160,10 @@ KVV_API int kvv_abi_version(void);
 /* Message of the last failed call on this thread ("" if none). */
 KVV_API const char* kvv_last_error(void);
 
-/* Workspace bytes kvv_verdict needs for this pair and policy. */
+/* Workspace bytes for this pair and policy.  They include a contiguous copy of
+ * each tensor (up to 1 GiB) whose layout rules out vector loads: a transposed or
+ * oddly sliced view is copied before the main pass.  kvv_verdict also runs,
+ * slower, with a workspace that has no room for the copies. */
 KVV_API int kvv_workspace_size(const kvv_tensor* gen, const kvv_tensor* ref, const kvv_policy* policy, size_t* bytes);
 
 /* One verdict: the data-parallel part of _compare_tensors

@@ -512,7 +512,7 @@ int launch_tail(const SegDesc* seg0, const SegDesc* dtable, const int64_t* dchun
   }
   if (nm.exact) {
     for (const auto& nl : nears) {
-      if (nl.items == 0) continue;
+      if (nl.items == 0) continue;  // (also a group without near-zero diagnostics)
       NearArgs na{};
       if (seg0) na.seg0 = *seg0;
       na.table = dtable ? dtable + nl.seg_lo : nullptr;
@@ -548,10 +548,33 @@ int launch_tail(const SegDesc* seg0, const SegDesc* dtable, const int64_t* dchun
 }
 
 // ------------------------------------------------------------ one verdict
-// A single pair too small to give every wave of the grid two full items takes
-// smaller items (down to one 16-byte vector per lane): more waves then share
-// its work, which for all-slow data is latency, not bandwidth.  The kernels
-// treat the vectors past an item's end as absent.
+// Items of fewer vectors per lane for work that leaves a grid's waves with few
+// full items each.  An item's time in a wave is mostly latency: about 6 parts of
+// staging, classification, samples and branches (5 us with a cold instruction
+// cache) to one part per vector, so the vector count taken is the one with the
+// least rounds x (6 + vectors), rounds = items per wave; the larger one on a tie.
+// The kernels treat the vectors past an item's end as absent.
+// `items_of(elems)`: the work's items at that item size.
+// (Two items of the smallest size that gives two, the earlier rule: 1 Mi fp32
+// elements took 71.6 us per verdict, 68.0 with one item of two vectors; 12 M bf16
+// elements 54.6 and 50.0.)
+template <typename F>
+int32_t item_size(int32_t full, F&& items_of) {
+  const int64_t waves = 3 * kWaves * (int64_t)device_cus();
+  int32_t best = full;
+  int64_t cost = -1;
+  for (int vec = kUnroll; vec >= 1; vec /= 2) {
+    const int32_t elems = full / kUnroll * vec;
+    const int64_t rounds = (items_of(elems) + waves - 1) / waves;
+    const int64_t c = rounds * (6 + vec);
+    if (cost < 0 || c < cost) {
+      cost = c;
+      best = elems;
+    }
+  }
+  return best;
+}
+
 int plan_single(const kvv_tensor* g, const kvv_tensor* r, const kvv_policy* p, SegDesc& d) {
   int rc = plan_segment(g, r, p, d);
   if (rc) return rc;
@@ -561,12 +584,8 @@ int plan_single(const kvv_tensor* g, const kvv_tensor* r, const kvv_policy* p, S
       scan_kind(d) != K_SCALAR)
     d.flags = (d.flags & ~KVV_FLAG_NEAR_ZERO) | kFlagNearEntries;
   if (scan_kind(d) == K_CONTIG) {
-    const int64_t min_elems = d.item_elems / kUnroll;
-    const int64_t want = 2 * 12 * (int64_t)device_cus();  // two items per wave of a full grid
-    while (d.item_elems > min_elems && d.item_count < want) {
-      d.item_elems /= 2;
-      d.item_count = (d.n + d.item_elems - 1) / d.item_elems;
-    }
+    d.item_elems = item_size(d.item_elems, [&](int32_t e) { return (d.n + e - 1) / e; });
+    d.item_count = (d.n + d.item_elems - 1) / d.item_elems;
   }
   return KVV_OK;
 }
@@ -1177,6 +1196,25 @@ int plan_batch(int32_t count, const kvv_tensor* gens, const kvv_tensor* refs, co
     }
   }
   auto key = [&](int i) { return (segs[i].dtype * 2 + segs[i].mode) * 3 + kinds[i]; };
+  // a group's contiguous pairs share an item size (item_size over the group's items)
+  {
+    int64_t total[kMaxGroups] = {}, pairs[kMaxGroups] = {};
+    for (int i = 0; i < count; ++i) {
+      total[key(i)] += segs[i].n;
+      ++pairs[key(i)];
+    }
+    int32_t elems[kMaxGroups] = {};
+    for (int i = 0; i < count; ++i) {
+      SegDesc& d = segs[i];
+      if (kinds[i] != K_CONTIG) continue;
+      int32_t& e = elems[key(i)];
+      // (each pair's last item counts as a whole one)
+      if (e == 0)
+        e = item_size(item_elems_for(d.dtype), [&](int32_t x) { return total[key(i)] / x + pairs[key(i)]; });
+      d.item_elems = e;
+      d.item_count = (d.n + e - 1) / e;
+    }
+  }
   std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return key(a) < key(b); });
   bp.table.clear();
   int64_t item = 0, sample = 0, chunk = 0;
@@ -1455,7 +1493,9 @@ int run_batch(BatchPlan& bp, kvv_result* out, void* ws, size_t ws_bytes, hipStre
   std::vector<NearLaunch> nears;
   bool zeroed = false;
   for (const auto& gr : bp.groups) {
-    nears.push_back({near_fn(gr.dt, gr.mode), gr.seg_lo, gr.seg_hi - gr.seg_lo, gr.item_lo, gr.items});
+    // (near-zero diagnostics exist for fp16 and bf16 pairs only, plan_segment)
+    const bool half = gr.dt == KVV_F16 || gr.dt == KVV_BF16;
+    nears.push_back({near_fn(gr.dt, gr.mode), gr.seg_lo, gr.seg_hi - gr.seg_lo, gr.item_lo, half ? gr.items : 0});
     if (gr.items == 0) continue;
     ScanFn scan = scan_fn(gr.dt, gr.mode, gr.kind, true);
     if (!scan) return fail(KVV_E_INVALID, "no kernel for dtype");

@@ -485,13 +485,23 @@ def release_buffers() -> None:
         _LAST[0] = None
 
 
-def _ensure(buf: _Buffers, dev: torch.device, ws_bytes: int, records: int) -> None:
-    """Grows buf's workspace and pinned record buffer to this call's needs (under buf.lock)."""
+# what any single pair's verdict runs with when the device has no room for the copies of its strided tensors
+_LEAST_WS = 64 << 20
+
+
+def _ensure(buf: _Buffers, dev: torch.device, ws_bytes: int, records: int, least: int = 0) -> None:
+    """Grows buf's workspace and pinned record buffer to this call's needs (under buf.lock).  With ``least``, a
+    device without ws_bytes free leaves a workspace of that size."""
     rec_size = ctypes.sizeof(_lib.KvvResult)
     if buf.ws is None or buf.ws.numel() < ws_bytes:
         buf.ws = None
         buf.kept = False
-        buf.ws = torch.empty(max(ws_bytes, 1 << 20), dtype=torch.uint8, device=dev)
+        try:
+            buf.ws = torch.empty(max(ws_bytes, 1 << 20), dtype=torch.uint8, device=dev)
+        except torch.OutOfMemoryError:
+            if not 0 < least < ws_bytes:
+                raise
+            buf.ws = torch.empty(least, dtype=torch.uint8, device=dev)
         buf.ws_bytes, buf.ws_ptr = buf.ws.numel(), buf.ws.data_ptr()
     if buf.out is None or buf.out.numel() < rec_size * records:
         # the records are written by the kernels straight into pinned host memory
@@ -554,7 +564,8 @@ def _launch_single(job: _Job) -> None:
                 plan[1].data = rp
             gt, rt, size = plan
             if buf.ws is None or buf.ws_bytes < size or buf.out is None:
-                _ensure(buf, torch.device("cuda", ri), size, 1)
+                _ensure(buf, torch.device("cuda", ri), size, 1, _LEAST_WS)
+                size = min(size, buf.ws_bytes)
             flags = kp.flags
             if buf.kept:
                 kp.flags = flags | _lib.FLAG_WS_KEPT
@@ -663,14 +674,15 @@ def _launch(jobs: List[_Job]) -> None:
             garr, rarr, parr = GA(*gts), GA(*rts), PA(*[j.kpolicy for j in jobs])
             _lib.check(lib.kvv_batch_workspace_size(n, garr, rarr, parr, ctypes.byref(size)), "kvv_batch_workspace_size")
         with buf.lock:
-            _ensure(buf, dev, size.value, n)
+            _ensure(buf, dev, size.value, n, _LEAST_WS if n == 1 else 0)
             ws, out = buf.ws, buf.out
             if n == 1:
                 pol = _lib.KvvPolicy.from_buffer_copy(jobs[0].kpolicy)
                 if buf.kept:
                     pol.flags |= _lib.FLAG_WS_KEPT
                 buf.kept = False  # (until this call has gone through)
-                rc = lib.kvv_verdict(gts[0], rts[0], pol, out.data_ptr(), ws.data_ptr(), size.value, stream)
+                rc = lib.kvv_verdict(gts[0], rts[0], pol, out.data_ptr(), ws.data_ptr(),
+                                     min(size.value, ws.numel()), stream)
                 _lib.check(rc, "kvv_verdict")
             else:
                 buf.kept = False

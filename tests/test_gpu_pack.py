@@ -122,3 +122,24 @@ def test_workspace_without_room_for_the_copies(shape):
         assert not record_vs_oracle(rec, g, r)
     exact = [k for k, v in recs[0].items() if isinstance(v, (int, list))] + ["p99_abs", "p99_rel", "max_abs", "max_rel"]
     assert all(recs[0][k] == recs[1][k] for k in exact)
+
+
+def test_device_without_room_for_the_copies(monkeypatch):
+    """A drop-in verdict whose workspace cannot be allocated with room for the copies runs with the least one."""
+    g, r = _pair((5000, 4100), torch.float32, 3)
+    gd, rd = g.to(DEV), _transposed(r.to(DEV))
+    want = verdict._compare_tensors(gd, rd, "output")
+    verdict.release_buffers()
+    empty = torch.empty
+
+    def short(n, *args, **kw):
+        if kw.get("dtype") == torch.uint8 and not kw.get("pin_memory") and n > verdict._LEAST_WS:
+            raise torch.OutOfMemoryError("no room")
+        return empty(n, *args, **kw)
+
+    monkeypatch.setattr(torch, "empty", short)
+    for _ in range(2):
+        assert repr(verdict._compare_tensors(gd, rd, "output")) == repr(want)
+    monkeypatch.undo()
+    assert repr(verdict._compare_tensors(gd, rd, "output")) == repr(want)
+    verdict.release_buffers()

@@ -770,7 +770,7 @@ __global__ __launch_bounds__(kBlock) void isel_cap_final_kernel(IselArgs a) {
     if (elems) cap_compact(a, d, nruns, x);
     const uint32_t r2[2] = {c.need[0] ? c.rk[0] : c.rk[1], c.need[1] ? c.rk[1] : c.rk[0]};
     uint32_t k[2];
-    range_keys(a.buf[x] + d.sample_off, cap[x], r2, k, L);
+    range_keys<false>(a.buf[x] + d.sample_off, cap[x], r2, k, L);
     // The main pass's dense items capture rel_diff from cap_rel_lo on, a few
     // roundings below the threshold: an order statistic from the threshold on
     // has every value that was not captured below it, a lower one may not

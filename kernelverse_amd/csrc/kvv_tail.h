@@ -787,6 +787,7 @@ __device__ inline bool small_keys(const float* v, int64_t count, const uint32_t 
   return has_nan;
 }
 
+template <bool SMALL>
 __device__ inline bool range_keys(const float* v, uint32_t count, const uint32_t rank[2], uint32_t key[2],
                                   SelectLds& L);
 
@@ -797,7 +798,7 @@ __device__ inline void select_small(const TailArgs& a, const SegDesc& d, int arr
   q99_ranks(count, rank64, wgt);
   const uint32_t rank[2] = {(uint32_t)rank64[0], (uint32_t)rank64[1]};
   uint32_t key[2];
-  const bool has_nan = range_keys(a.arr[arr] + d.sample_off, (uint32_t)count, rank, key, L);
+  const bool has_nan = range_keys<true>(a.arr[arr] + d.sample_off, (uint32_t)count, rank, key, L);
   finalize_group(a, d, arr, count, key, wgt, has_nan, L);
 }
 
@@ -928,13 +929,27 @@ __device__ inline bool stream_keys(const float* v, int64_t count, const uint32_t
 // narrow range (e.g. the top few percent of a distribution, whose leading key
 // bits agree) thus spread over the bins instead of meeting in a few LDS words.
 // Values stay in registers when there are at most kSmall of them, else every
-// pass reads them again.  Returns whether a value is NaN (the keys are then
-// not searched).  Called by all threads of the block.
+// pass reads them again.
+// SMALL (a small group of a tail launch, at most kSmall values): as soon as the
+// ranks' bins hold at most kCand values, those are collected in LDS and ranked
+// there by comparing all pairs (usual after the first pass: a rank's bin of
+// 4,096 noise differences holds about 30), one light pass over the values
+// instead of two or three with histograms.  Such a block runs once, from a cold
+// instruction cache, so the first pass, whose two ranks share one range, has
+// code of its own.  The tail launch of a 4,096-element fp32 pair: 18.5 -> 12.8
+// us, its verdict 48.9 -> 43.5.  Not for the capture final's lists: their bins
+// hold hundreds of values and its blocks share the CUs (five waves per SIMD);
+// with the candidates it took 171 us instead of 150 (4,096 ragged pairs), as one
+// function of 147 VGPRs 257.
+// Returns whether a value is NaN (the keys are then not searched).  Called by
+// all threads of the block.
+constexpr uint32_t kCand = kBlock;
+template <bool SMALL>
 __device__ inline bool range_keys(const float* v, uint32_t count, const uint32_t rank[2], uint32_t key[2],
                                   SelectLds& L) {
   constexpr int PER = kSmall / kBlock;
   const int tid = threadIdx.x;
-  const bool regs = count <= (uint32_t)kSmall;
+  const bool regs = SMALL || count <= (uint32_t)kSmall;
   uint32_t k[PER];
 #pragma unroll
   for (int i = 0; i < PER; ++i) {
@@ -944,9 +959,14 @@ __device__ inline bool range_keys(const float* v, uint32_t count, const uint32_t
   // f(key) for every value of this thread
   auto visit = [&](auto&& f) {
     if (regs) {
+      // (SMALL: eight at a time, the code of the absent ones is not even fetched)
 #pragma unroll
-      for (int i = 0; i < PER; ++i)
-        if ((uint32_t)(i * kBlock + tid) < count) f(k[i]);
+      for (int g = 0; g < PER; g += 8) {
+        if (SMALL && (uint32_t)(g * kBlock) >= count) break;
+#pragma unroll
+        for (int i = g; i < g + 8; ++i)
+          if ((uint32_t)(i * kBlock + tid) < count) f(k[i]);
+      }
     } else {
       // eight loads in flight per thread
       for (uint32_t i0 = 0; i0 < count; i0 += 8 * kBlock) {
@@ -972,23 +992,24 @@ __device__ inline bool range_keys(const float* v, uint32_t count, const uint32_t
   key[0] = key[1] = 0u;
   // NaNs and exact zeros counted together (each at most the block's count, below 2^16 when
   // the values are in registers; else only the NaN count is used)
-  const uint32_t nz = block_sum_nan(regs ? nans | (zeros << 16) : nans, L);
-  if ((regs ? nz & 0xFFFFu : nz) != 0) return true;
+  const uint32_t nzw = wave_sum(regs ? nans | (zeros << 16) : nans);
   mn = wave_min(mn);
   mx = wave_max(mx);
+  __syncthreads();
   if ((tid & 63) == 0) {
-    L.misc[tid >> 6] = mn;
-    L.sh[tid >> 6] = mx;
+    L.sh[tid >> 6] = mn;
+    L.sh[kWaves + (tid >> 6)] = mx;
+    L.misc[tid >> 6] = nzw;
   }
   __syncthreads();
-  mn = L.misc[0];
-  mx = L.sh[0];
+  uint32_t nz = 0;
 #pragma unroll
-  for (int w = 1; w < kWaves; ++w) {
-    mn = L.misc[w] < mn ? L.misc[w] : mn;
-    mx = L.sh[w] > mx ? L.sh[w] : mx;
+  for (int w = 0; w < kWaves; ++w) {
+    mn = L.sh[w] < mn ? L.sh[w] : mn;
+    mx = L.sh[kWaves + w] > mx ? L.sh[kWaves + w] : mx;
+    nz += L.misc[w];
   }
-  __syncthreads();
+  if ((regs ? nz & 0xFFFFu : nz) != 0) return true;
   // both ranks among the exact zeros, the least values (the p99 of mostly identical pairs): no pass
   if (regs && mn == kZeroKey && rank[1] < (nz >> 16)) {
     key[0] = key[1] = kZeroKey;
@@ -1005,36 +1026,42 @@ __device__ inline bool range_keys(const float* v, uint32_t count, const uint32_t
       const int bits = 32 - __clz(hi[t] - lo[t]);
       shift[t] = bits > 11 ? bits - 11 : 0;
     }
-    for (int i = tid; i < 2 * 2048; i += kBlock) (&L.h[0][0])[i] = 0;
+    const bool both = lo[0] != hi[0] && lo[1] != hi[1];
+    for (int i = tid; i < (same ? 2048 : 2 * 2048); i += kBlock) (&L.h[0][0])[i] = 0;
+    if (tid == 0) L.sh[14] = 0;  // (collected candidates)
     __syncthreads();
     // a lane's consecutive values of one bin are added once (repeated values,
     // e.g. the zeros of mostly identical data, would serialise on one word)
-    uint32_t rb[2] = {0u, 0u}, rn[2] = {0u, 0u};
-    visit([&](uint32_t kk) {
-#pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        if ((t == 0 || !same) && lo[t] != hi[t] && kk >= lo[t] && kk <= hi[t]) {
-          const uint32_t bin = (kk - lo[t]) >> shift[t];
-          if (bin != rb[t]) {
-            if (rn[t]) atomicAdd(&L.h[t][rb[t]], rn[t]);
-            rb[t] = bin;
-            rn[t] = 0;
-          }
-          ++rn[t];
+    uint32_t rbA = 0u, rnA = 0u, rbB = 0u, rnB = 0u;
+    auto add = [](uint32_t* h, uint32_t kk, uint32_t from, uint32_t to, int sh, uint32_t& rb, uint32_t& rn) {
+      if (from != to && kk >= from && kk <= to) {
+        const uint32_t bin = (kk - from) >> sh;
+        if (bin != rb) {
+          if (rn) atomicAdd(&h[rb], rn);
+          rb = bin;
+          rn = 0;
         }
+        ++rn;
       }
-    });
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-      if (rn[t]) atomicAdd(&L.h[t][rb[t]], rn[t]);
+    };
+    if (SMALL && same) {
+      visit([&](uint32_t kk) { add(L.h[0], kk, lo[0], hi[0], shift[0], rbA, rnA); });
+    } else {
+      visit([&](uint32_t kk) {
+        add(L.h[0], kk, lo[0], hi[0], shift[0], rbA, rnA);
+        if (!same) add(L.h[1], kk, lo[1], hi[1], shift[1], rbB, rnB);
+      });
+    }
+    if (rnA) atomicAdd(&L.h[0][rbA], rnA);
+    if (rnB) atomicAdd(&L.h[1][rbB], rnB);
     __syncthreads();
-    uint32_t cA[8], cB[8], bin[2], below[2];
+    uint32_t cA[8], cB[8], bin[2], below[2], cnt[2] = {0u, 0u};
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       cA[i] = L.h[0][tid * 8 + i];
       cB[i] = L.h[1][tid * 8 + i];
     }
-    block_find2<8>(cA, cB, same, resid, bin, below, L.sh);
+    block_find2<8>(cA, cB, same, resid, bin, below, L.sh, SMALL ? cnt : nullptr);
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
       if (lo[t] == hi[t]) continue;
@@ -1043,6 +1070,38 @@ __device__ inline bool range_keys(const float* v, uint32_t count, const uint32_t
       lo[t] = (uint32_t)nlo;
       hi[t] = nhi < hi[t] ? (uint32_t)nhi : hi[t];
       resid[t] -= below[t];
+    }
+    // (both ranges now hold cnt values each, the same ones or the second's all above the first's)
+    const bool one = lo[0] == lo[1];
+    const uint32_t n = cnt[0] + (one ? 0u : cnt[1]);
+    if (SMALL && both && n <= kCand && !(lo[0] == hi[0] && lo[1] == hi[1])) {
+      uint32_t* const cand = reinterpret_cast<uint32_t*>(L.part);
+      const uint32_t r0 = hi[0] - lo[0], r1 = hi[1] - lo[1];
+      visit([&](uint32_t kk) {
+        if (kk - lo[0] <= r0 || kk - lo[1] <= r1) {
+          const uint32_t p = atomicAdd(&L.sh[14], 1u);
+          if (p < kCand) cand[p] = kk;
+        }
+      });
+      if (tid == 0 && (n & 1u)) cand[n] = 0xFFFFFFFFu;  // (the last word pair's absent value; n odd: below kCand)
+      __syncthreads();
+      if ((uint32_t)tid < n) {
+        const uint32_t q0 = resid[0], q1 = one ? resid[1] : cnt[0] + resid[1], my = cand[tid];
+        const uint2* const c2 = reinterpret_cast<const uint2*>(L.part);
+        uint32_t less = 0, le = 0;
+#pragma unroll 4
+        for (uint32_t j = 0; j < (n + 1) / 2; ++j) {
+          const uint2 c = c2[j];
+          less += (c.x < my ? 1u : 0u) + (c.y < my ? 1u : 0u);
+          le += (c.x <= my ? 1u : 0u) + (c.y <= my ? 1u : 0u);
+        }
+        if (less <= q0 && q0 < le) L.sh[8] = my;
+        if (less <= q1 && q1 < le) L.sh[9] = my;
+      }
+      __syncthreads();
+      key[0] = L.sh[8];
+      key[1] = L.sh[9];
+      return false;
     }
     __syncthreads();
   }

@@ -548,7 +548,8 @@ def _launch_single(job: _Job) -> None:
         buf = _stream_buffers(_cuda_device(ri))
         kp = job.kpolicy
         gp, rp = g.data_ptr(), r.data_ptr()
-        key = (job.pkey, g.dtype, g.shape, g.stride(), r.stride(), (gp & 15) == 0, (rp & 15) == 0)
+        # (both tensors' types and shapes: a pair that differs in them has no plan, and planning refuses it)
+        key = (job.pkey, g.dtype, r.dtype, g.shape, r.shape, g.stride(), r.stride(), (gp & 15) == 0, (rp & 15) == 0)
         with buf.lock:
             plan = buf.plans.get(key)
             if plan is None:
@@ -600,7 +601,8 @@ def _launch_planned(jobs: List[_Job]) -> bool:
             return False
         gp, rp = g.data_ptr(), r.data_ptr()
         ptrs.append((gp, rp))
-        key.append((j.pkey, g.dtype, g.shape, g.stride(), r.stride(), (gp & 15) == 0, (rp & 15) == 0))
+        # (both tensors' types and shapes: a pair that differs in them has no plan, and planning refuses it)
+        key.append((j.pkey, g.dtype, r.dtype, g.shape, r.shape, g.stride(), r.stride(), (gp & 15) == 0, (rp & 15) == 0))
     key = tuple(key)
     lib = _lib.load()
     n = len(jobs)

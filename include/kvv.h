@@ -166,6 +166,12 @@ KVV_API const char* kvv_last_error(void);
  * slower, with a workspace that has no room for the copies. */
 KVV_API int kvv_workspace_size(const kvv_tensor* gen, const kvv_tensor* ref, const kvv_policy* policy, size_t* bytes);
 
+/* What that size holds: `least`, the bytes kvv_verdict runs this pair with at all
+ * (no copies, the smallest near-zero entry pool), and `copies`, the bytes of it
+ * that are copies of the tensors (0: none). */
+KVV_API int kvv_workspace_parts(const kvv_tensor* gen, const kvv_tensor* ref, const kvv_policy* policy, size_t* least,
+                                size_t* copies);
+
 /* One verdict: the data-parallel part of _compare_tensors
  * (generated_correctness_runner.py:672-786) for one tensor pair.
  *   gen, ref    same shape and dtype (checked; the reference returns a

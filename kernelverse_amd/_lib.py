@@ -111,8 +111,8 @@ class KvvResult(ctypes.Structure):
         return out
 
 
-EXPORTED = ("kvv_abi_version", "kvv_last_error", "kvv_workspace_size", "kvv_verdict", "kvv_verdict_timed",
-            "kvv_verdict_noalloc", "kvv_batch_workspace_size", "kvv_verdict_batch")
+EXPORTED = ("kvv_abi_version", "kvv_last_error", "kvv_workspace_size", "kvv_workspace_parts", "kvv_verdict",
+            "kvv_verdict_timed", "kvv_verdict_noalloc", "kvv_batch_workspace_size", "kvv_verdict_batch")
 
 # the fixed workspace of kvv_verdict_noalloc (bytes)
 NOALLOC_SCRATCH_BYTES = 64 << 20
@@ -138,6 +138,9 @@ def load() -> ctypes.CDLL:
     lib.kvv_last_error.argtypes = []
     lib.kvv_workspace_size.restype = c_int32
     lib.kvv_workspace_size.argtypes = [POINTER(KvvTensor), POINTER(KvvTensor), POINTER(KvvPolicy), POINTER(c_size_t)]
+    lib.kvv_workspace_parts.restype = c_int32
+    lib.kvv_workspace_parts.argtypes = [POINTER(KvvTensor), POINTER(KvvTensor), POINTER(KvvPolicy), POINTER(c_size_t),
+                                        POINTER(c_size_t)]
     lib.kvv_verdict.restype = c_int32
     lib.kvv_verdict.argtypes = [POINTER(KvvTensor), POINTER(KvvTensor), POINTER(KvvPolicy), c_void_p, c_void_p,
                                 c_size_t, c_void_p]

@@ -1606,6 +1606,19 @@ int kvv_workspace_size(const kvv_tensor* gen, const kvv_tensor* ref, const kvv_p
   return KVV_OK;
 }
 
+int kvv_workspace_parts(const kvv_tensor* gen, const kvv_tensor* ref, const kvv_policy* policy, size_t* least,
+                        size_t* copies) {
+  if (!least || !copies) return kvv::fail(KVV_E_INVALID, "null size pointer");
+  kvv::SegDesc d;
+  int rc = kvv::plan_single(gen, ref, policy, d);
+  if (rc) return rc;
+  rc = kvv::single_workspace_bytes(d, least, false);
+  if (rc) return rc;
+  kvv::PackPlan pp;
+  *copies = kvv::plan_pack(gen, ref, policy, d, pp) ? pp.total - pp.base : 0;
+  return KVV_OK;
+}
+
 int kvv_verdict(const kvv_tensor* gen, const kvv_tensor* ref, const kvv_policy* policy, kvv_result* out,
                 void* workspace, size_t workspace_bytes, void* stream) {
   return kvv::run_pair(gen, ref, policy, out, workspace, workspace_bytes, static_cast<hipStream_t>(stream),

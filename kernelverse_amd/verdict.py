@@ -485,29 +485,45 @@ def release_buffers() -> None:
         _LAST[0] = None
 
 
-# what any single pair's verdict runs with when the device has no room for the copies of its strided tensors
+# a device without room for a pair's full workspace gives this much, where the pair runs in it, before the least one
 _LEAST_WS = 64 << 20
 
 
-def _ensure(buf: _Buffers, dev: torch.device, ws_bytes: int, records: int, least: int = 0) -> None:
-    """Grows buf's workspace and pinned record buffer to this call's needs (under buf.lock).  With ``least``, a
-    device without ws_bytes free leaves a workspace of that size."""
+def _ensure(buf: _Buffers, dev: torch.device, ws_bytes: int, records: int) -> None:
+    """Grows buf's workspace and pinned record buffer to this call's needs (under buf.lock)."""
     rec_size = ctypes.sizeof(_lib.KvvResult)
     if buf.ws is None or buf.ws.numel() < ws_bytes:
         buf.ws = None
         buf.kept = False
-        try:
-            buf.ws = torch.empty(max(ws_bytes, 1 << 20), dtype=torch.uint8, device=dev)
-        except torch.OutOfMemoryError:
-            if not 0 < least < ws_bytes:
-                raise
-            buf.ws = torch.empty(least, dtype=torch.uint8, device=dev)
+        buf.ws = torch.empty(max(ws_bytes, 1 << 20), dtype=torch.uint8, device=dev)
         buf.ws_bytes, buf.ws_ptr = buf.ws.numel(), buf.ws.data_ptr()
     if buf.out is None or buf.out.numel() < rec_size * records:
         # the records are written by the kernels straight into pinned host memory
         buf.out = torch.empty(max(rec_size * records, 64 * rec_size), dtype=torch.uint8, pin_memory=True)
         buf.out_ptr = buf.out.data_ptr()
         buf.out_rec = (ctypes.c_char * rec_size).from_address(buf.out_ptr)
+
+
+def _room(buf: _Buffers, dev: torch.device, gt, rt, kp, size: int):
+    """buf's workspace for one pair whose kvv_workspace_size is ``size``, under buf.lock: (pointer, bytes).
+
+    Where the device has no room for the whole, the pair runs in less, down to the least its verdict
+    needs (no copies: the scalar pass)."""
+    if buf.ws is not None and buf.ws_bytes >= size:
+        _ensure(buf, dev, 0, 1)
+        return buf.ws_ptr, size
+    least, copies = ctypes.c_size_t(), ctypes.c_size_t()
+    _lib.check(_lib.load().kvv_workspace_parts(gt, rt, kp, ctypes.byref(least), ctypes.byref(copies)),
+               "kvv_workspace_parts")
+    least = least.value
+    tries = [size] + [s for s in (_LEAST_WS, least) if least <= s < size]
+    for s in tries:
+        try:
+            _ensure(buf, dev, s, 1)
+            return buf.ws_ptr, min(size, buf.ws_bytes)
+        except torch.OutOfMemoryError:
+            if s == tries[-1]:
+                raise
 
 
 def _device_of(job: _Job) -> torch.device:
@@ -564,15 +580,15 @@ def _launch_single(job: _Job) -> None:
                 plan[0].data = gp
                 plan[1].data = rp
             gt, rt, size = plan
+            ws = buf.ws_ptr
             if buf.ws is None or buf.ws_bytes < size or buf.out is None:
-                _ensure(buf, torch.device("cuda", ri), size, 1, _LEAST_WS)
-                size = min(size, buf.ws_bytes)
+                ws, size = _room(buf, _cuda_device(ri), gt, rt, kp, size)
             flags = kp.flags
             if buf.kept:
                 kp.flags = flags | _lib.FLAG_WS_KEPT
             buf.kept = False  # (until this call has gone through)
             try:
-                rc = lib.kvv_verdict(gt, rt, kp, buf.out_ptr, buf.ws_ptr, size, buf.handle)
+                rc = lib.kvv_verdict(gt, rt, kp, buf.out_ptr, ws, size, buf.handle)
             finally:
                 kp.flags = flags
             _lib.check(rc, "kvv_verdict")
@@ -676,23 +692,22 @@ def _launch(jobs: List[_Job]) -> None:
             garr, rarr, parr = GA(*gts), GA(*rts), PA(*[j.kpolicy for j in jobs])
             _lib.check(lib.kvv_batch_workspace_size(n, garr, rarr, parr, ctypes.byref(size)), "kvv_batch_workspace_size")
         with buf.lock:
-            _ensure(buf, dev, size.value, n, _LEAST_WS if n == 1 else 0)
-            ws, out = buf.ws, buf.out
             if n == 1:
+                ws, ws_bytes = _room(buf, dev, gts[0], rts[0], jobs[0].kpolicy, size.value)
                 pol = _lib.KvvPolicy.from_buffer_copy(jobs[0].kpolicy)
                 if buf.kept:
                     pol.flags |= _lib.FLAG_WS_KEPT
                 buf.kept = False  # (until this call has gone through)
-                rc = lib.kvv_verdict(gts[0], rts[0], pol, out.data_ptr(), ws.data_ptr(),
-                                     min(size.value, ws.numel()), stream)
+                rc = lib.kvv_verdict(gts[0], rts[0], pol, buf.out_ptr, ws, ws_bytes, stream)
                 _lib.check(rc, "kvv_verdict")
             else:
+                _ensure(buf, dev, size.value, n)
                 buf.kept = False
-                rc = lib.kvv_verdict_batch(n, garr, rarr, parr, out.data_ptr(), ws.data_ptr(), size.value, stream)
+                rc = lib.kvv_verdict_batch(n, garr, rarr, parr, buf.out_ptr, buf.ws_ptr, size.value, stream)
                 _lib.check(rc, "kvv_verdict_batch")
             buf.stream.synchronize()
             buf.kept = True
-            host = ctypes.string_at(out.data_ptr(), rec_size * n)
+            host = ctypes.string_at(buf.out_ptr, rec_size * n)
     finally:
         if ctx is not None:
             ctx.__exit__(None, None, None)

@@ -412,7 +412,7 @@ class _Buffers:
     output (at most ``_MAX_BATCH_PAIRS`` of them)."""
 
     __slots__ = ("lock", "ws", "out", "kept", "stream", "handle", "plans", "batch_plans", "ws_bytes", "ws_ptr",
-                 "out_ptr", "out_rec")
+                 "out_ptr", "out_rec", "short_bytes", "short_calls")
 
     def __init__(self, stream):
         self.lock = threading.Lock()
@@ -425,6 +425,7 @@ class _Buffers:
         self.batch_plans: "OrderedDict[tuple, tuple]" = OrderedDict()
         self.ws_bytes = self.ws_ptr = self.out_ptr = 0
         self.out_rec = None  # the first record's bytes in `out`, as a ctypes view
+        self.short_bytes = self.short_calls = 0  # the last size that found no room, and how long it is not tried
 
 
 _MAX_STREAMS = 8
@@ -487,6 +488,8 @@ def release_buffers() -> None:
 
 # a device without room for a pair's full workspace gives this much, where the pair runs in it, before the least one
 _LEAST_WS = 64 << 20
+# verdicts whose workspace is at least as large as one that found no room run in less for this many calls
+_SHORT_CALLS = 64
 
 
 def _ensure(buf: _Buffers, dev: torch.device, ws_bytes: int, records: int) -> None:
@@ -508,7 +511,7 @@ def _room(buf: _Buffers, dev: torch.device, gt, rt, kp, size: int):
     """buf's workspace for one pair whose kvv_workspace_size is ``size``, under buf.lock: (pointer, bytes).
 
     Where the device has no room for the whole, the pair runs in less, down to the least its verdict
-    needs (no copies: the scalar pass)."""
+    needs (no copies: the scalar pass), and the next calls do not ask for as much again."""
     if buf.ws is not None and buf.ws_bytes >= size:
         _ensure(buf, dev, 0, 1)
         return buf.ws_ptr, size
@@ -517,6 +520,9 @@ def _room(buf: _Buffers, dev: torch.device, gt, rt, kp, size: int):
                "kvv_workspace_parts")
     least = least.value
     tries = [size] + [s for s in (_LEAST_WS, least) if least <= s < size]
+    if buf.short_calls and size >= buf.short_bytes and len(tries) > 1:
+        buf.short_calls -= 1
+        del tries[0]
     for s in tries:
         try:
             _ensure(buf, dev, s, 1)
@@ -524,6 +530,8 @@ def _room(buf: _Buffers, dev: torch.device, gt, rt, kp, size: int):
         except torch.OutOfMemoryError:
             if s == tries[-1]:
                 raise
+            if s == size:
+                buf.short_bytes, buf.short_calls = size, _SHORT_CALLS
 
 
 def _device_of(job: _Job) -> torch.device:

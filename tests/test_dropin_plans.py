@@ -5,7 +5,7 @@ recorders and device allocations by plain sizes with a limit.
 * A pair whose tensors differ in shape or type is refused before anything is
   launched, whatever plans earlier calls left.
 * A pair whose workspace holds copies of its tensors runs without them where the
-  device has no room."""
+  device has no room, and does not ask for that room again on each call."""
 
 import ctypes
 
@@ -133,13 +133,14 @@ def _transposed(rows, cols):
 
 @pytest.mark.parametrize("max_samples,room", [(1_000_000, 64 << 20), (1 << 24, 200 << 20)])
 def test_device_without_room_for_the_copies(device, max_samples, room):
-    """The fallback holds the pair's own samples (2 x 64 MiB at the largest max_samples)."""
+    """The fallback holds the pair's own samples (2 x 64 MiB at the largest max_samples), and the size that found no
+    room is asked for again only after _SHORT_CALLS calls."""
     pair = _transposed(5000, 4100)
     device.room = room
-    for _ in range(2):
+    for _ in range(1 + verdict._SHORT_CALLS):
         verdict.verdict_records([pair], max_samples=max_samples)
     full = max(device.asked)
-    assert full > room
+    assert full > room and device.asked.count(full) == 1
     assert all(b <= room for _, b in device.lib.launched)
     device.room = 1 << 50
     verdict.verdict_records([pair], max_samples=max_samples)

@@ -400,9 +400,9 @@ class _Buffers:
 
     Every call synchronises its stream before it returns, so consecutive calls
     on one stream can reuse both; the lock serialises threads that share the
-    stream.  Each grows to the largest call seen.  At most ``_MAX_STREAMS``
-    (device, stream) entries are kept: a new stream evicts the least recently
-    used idle one, and ``release_buffers`` frees them all.
+    stream.  Each grows to the largest call seen (large copies aside, ``_room``).
+    At most ``_MAX_STREAMS`` (device, stream) entries are kept: a new stream
+    evicts the least recently used idle one, and ``release_buffers`` frees them all.
     ``kept``: the workspace went through a previous call and nothing else writes
     it, so single-pair calls pass KVV_FLAG_WS_KEPT (the library then skips
     clearing the select slots that call left clear).
@@ -488,6 +488,8 @@ def release_buffers() -> None:
 
 # a device without room for a pair's full workspace gives this much, where the pair runs in it, before the least one
 _LEAST_WS = 64 << 20
+# a workspace above this because of its tensors' copies is the call's own: it goes back to the allocator afterwards
+_KEPT_COPIES = 256 << 20
 # verdicts whose workspace is at least as large as one that found no room run in less for this many calls
 _SHORT_CALLS = 64
 
@@ -508,13 +510,15 @@ def _ensure(buf: _Buffers, dev: torch.device, ws_bytes: int, records: int) -> No
 
 
 def _room(buf: _Buffers, dev: torch.device, gt, rt, kp, size: int):
-    """buf's workspace for one pair whose kvv_workspace_size is ``size``, under buf.lock: (pointer, bytes).
+    """A workspace for one pair whose kvv_workspace_size is ``size``, under buf.lock: (pointer, bytes, tensor), the
+    tensor None for buf's own.
 
-    Where the device has no room for the whole, the pair runs in less, down to the least its verdict
+    Copies that take it above ``_KEPT_COPIES`` are not kept: up to 1 GiB per tensor for every stream would stay
+    reserved.  Where the device has no room for the whole, the pair runs in less, down to the least its verdict
     needs (no copies: the scalar pass), and the next calls do not ask for as much again."""
     if buf.ws is not None and buf.ws_bytes >= size:
         _ensure(buf, dev, 0, 1)
-        return buf.ws_ptr, size
+        return buf.ws_ptr, size, None
     least, copies = ctypes.c_size_t(), ctypes.c_size_t()
     _lib.check(_lib.load().kvv_workspace_parts(gt, rt, kp, ctypes.byref(least), ctypes.byref(copies)),
                "kvv_workspace_parts")
@@ -525,8 +529,12 @@ def _room(buf: _Buffers, dev: torch.device, gt, rt, kp, size: int):
         del tries[0]
     for s in tries:
         try:
+            if s == size and copies.value and size > _KEPT_COPIES:
+                own = torch.empty(size, dtype=torch.uint8, device=dev)
+                _ensure(buf, dev, 0, 1)
+                return own.data_ptr(), size, own
             _ensure(buf, dev, s, 1)
-            return buf.ws_ptr, min(size, buf.ws_bytes)
+            return buf.ws_ptr, min(size, buf.ws_bytes), None
         except torch.OutOfMemoryError:
             if s == tries[-1]:
                 raise
@@ -588,13 +596,16 @@ def _launch_single(job: _Job) -> None:
                 plan[0].data = gp
                 plan[1].data = rp
             gt, rt, size = plan
-            ws = buf.ws_ptr
+            ws, own = buf.ws_ptr, None
             if buf.ws is None or buf.ws_bytes < size or buf.out is None:
-                ws, size = _room(buf, _cuda_device(ri), gt, rt, kp, size)
+                ws, size, own = _room(buf, _cuda_device(ri), gt, rt, kp, size)
             flags = kp.flags
-            if buf.kept:
-                kp.flags = flags | _lib.FLAG_WS_KEPT
-            buf.kept = False  # (until this call has gone through)
+            kept = buf.kept
+            if own is None:
+                if kept:
+                    kp.flags = flags | _lib.FLAG_WS_KEPT
+                buf.kept = False  # (until this call has gone through)
+                kept = True
             try:
                 rc = lib.kvv_verdict(gt, rt, kp, buf.out_ptr, ws, size, buf.handle)
             finally:
@@ -603,7 +614,7 @@ def _launch_single(job: _Job) -> None:
             # host work that needs no record, done while the device runs
             job.tol_text = f"{job.tolerance}"
             buf.stream.synchronize()
-            buf.kept = True
+            buf.kept = kept
             job.record = _lib.KvvResult.from_buffer_copy(buf.out_rec)
     finally:
         if ctx is not None:
@@ -700,12 +711,16 @@ def _launch(jobs: List[_Job]) -> None:
             garr, rarr, parr = GA(*gts), GA(*rts), PA(*[j.kpolicy for j in jobs])
             _lib.check(lib.kvv_batch_workspace_size(n, garr, rarr, parr, ctypes.byref(size)), "kvv_batch_workspace_size")
         with buf.lock:
+            kept = True
             if n == 1:
-                ws, ws_bytes = _room(buf, dev, gts[0], rts[0], jobs[0].kpolicy, size.value)
+                ws, ws_bytes, own = _room(buf, dev, gts[0], rts[0], jobs[0].kpolicy, size.value)
                 pol = _lib.KvvPolicy.from_buffer_copy(jobs[0].kpolicy)
-                if buf.kept:
-                    pol.flags |= _lib.FLAG_WS_KEPT
-                buf.kept = False  # (until this call has gone through)
+                if own is None:
+                    if buf.kept:
+                        pol.flags |= _lib.FLAG_WS_KEPT
+                    buf.kept = False  # (until this call has gone through)
+                else:
+                    kept = buf.kept
                 rc = lib.kvv_verdict(gts[0], rts[0], pol, buf.out_ptr, ws, ws_bytes, stream)
                 _lib.check(rc, "kvv_verdict")
             else:
@@ -714,7 +729,7 @@ def _launch(jobs: List[_Job]) -> None:
                 rc = lib.kvv_verdict_batch(n, garr, rarr, parr, buf.out_ptr, buf.ws_ptr, size.value, stream)
                 _lib.check(rc, "kvv_verdict_batch")
             buf.stream.synchronize()
-            buf.kept = True
+            buf.kept = kept
             host = ctypes.string_at(buf.out_ptr, rec_size * n)
     finally:
         if ctx is not None:

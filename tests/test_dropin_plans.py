@@ -5,7 +5,8 @@ recorders and device allocations by plain sizes with a limit.
 * A pair whose tensors differ in shape or type is refused before anything is
   launched, whatever plans earlier calls left.
 * A pair whose workspace holds copies of its tensors runs without them where the
-  device has no room, and does not ask for that room again on each call."""
+  device has no room, does not ask for that room again on each call, and keeps no
+  large copies between calls."""
 
 import ctypes
 
@@ -153,3 +154,14 @@ def test_contiguous_pair_without_room_raises(device):
     with pytest.raises(torch.OutOfMemoryError):
         verdict.verdict_records([(g, g)])
     assert device.lib.launched == []
+
+
+def test_large_copies_are_not_kept(device):
+    small, large = _transposed(2000, 3000), _transposed(16384, 16384)
+    verdict.verdict_records([small])
+    held = device.buf.ws_bytes
+    for _ in range(2):
+        verdict.verdict_records([large])
+        assert device.lib.launched[-1][1] > 1 << 30 and device.buf.ws_bytes == held and device.buf.kept
+    verdict.verdict_records([small])
+    assert device.lib.launched[-1][1] <= held

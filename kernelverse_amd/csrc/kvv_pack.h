@@ -28,6 +28,11 @@ namespace kvv {
 
 constexpr int kPackTile = 64;
 
+// Tensors above this many bytes are not packed: the copies would cost that much
+// workspace each.
+constexpr int64_t kPackMax = int64_t(1) << 30;
+static_assert(kPackMax < (int64_t(1) << 31), "32-bit element indices and block counts");
+
 struct PackArgs {
   const void* src;
   void* dst;
@@ -54,29 +59,21 @@ __global__ __launch_bounds__(256) void pack_gather_kernel(PackArgs a) {
   if (i0 >= a.n) return;
   const T* src = reinterpret_cast<const T*>(a.src);
   T* dst = reinterpret_cast<T*>(a.dst);
-  // the first element's index, innermost dim last
-  int64_t off = 0, c_last = 0;
-  if (((uint64_t)a.n >> 32) == 0) {
-    uint32_t r = (uint32_t)i0;
+  // source offset of element i; c: its index in the innermost dim
+  auto offset_of = [&](uint32_t i, uint32_t& c) {
+    int64_t off = 0;
+    uint32_t r = i;
+    c = r;
     for (int k = a.nd - 1; k > 0; --k) {
-      const uint32_t s = (uint32_t)a.sizes[k], q = r / s, c = r - q * s;
-      if (k == a.nd - 1) c_last = c;
-      off += (int64_t)c * a.str[k];
+      const uint32_t s = (uint32_t)a.sizes[k], q = r / s, x = r - q * s;
+      if (k == a.nd - 1) c = x;
+      off += (int64_t)x * a.str[k];
       r = q;
     }
-    if (a.nd == 1) c_last = r;
-    off += (int64_t)r * a.str[0];
-  } else {
-    int64_t r = i0;
-    for (int k = a.nd - 1; k > 0; --k) {
-      const int64_t q = r / a.sizes[k], c = r - q * a.sizes[k];
-      if (k == a.nd - 1) c_last = c;
-      off += c * a.str[k];
-      r = q;
-    }
-    if (a.nd == 1) c_last = r;
-    off += r * a.str[0];
-  }
+    return off + (int64_t)r * a.str[0];
+  };
+  uint32_t c_last;
+  const int64_t off = offset_of((uint32_t)i0, c_last);
   const int64_t s_last = a.str[a.nd - 1];
   const int ne = a.n - i0 < V ? (int)(a.n - i0) : V;
   if (ne == V && c_last + V <= a.sizes[a.nd - 1]) {
@@ -86,15 +83,7 @@ __global__ __launch_bounds__(256) void pack_gather_kernel(PackArgs a) {
     return;
   }
   // a vector across rows, or the tensor's last
-  for (int e = 0; e < ne; ++e) {
-    int64_t r = i0 + e, at = 0;
-    for (int k = a.nd - 1; k > 0; --k) {
-      const int64_t q = r / a.sizes[k];
-      at += (r - q * a.sizes[k]) * a.str[k];
-      r = q;
-    }
-    dst[i0 + e] = src[at + r * a.str[0]];
-  }
+  for (int e = 0; e < ne; ++e) dst[i0 + e] = src[offset_of((uint32_t)(i0 + e), c_last)];
 }
 
 template <typename T>

@@ -1331,22 +1331,23 @@ __device__ __forceinline__ bool phase_b_dense(const SegDesc& d, uint32_t R0, uin
 
 // ------------------------------------------------------------ dense items
 // An item in which many pairs differ (fp32 results that differ by rounding
-// noise everywhere, 16-bit results that round elsewhere), for the isclose test
-// of fp32, bf16 and fp16: every lane finishes its own stage slots in order,
+// noise everywhere, 16-bit results that round elsewhere) and most of those within
+// the tolerance (dense_pays), for the isclose test of fp32, bf16 and fp16: every
+// lane finishes its own stage slots in order,
 // the bit-identical pairs among them, so neither phase A's classification nor
 // the queue is needed.  Only the outputs that every pair has are taken per
 // element: the fp64 products, the ULP bucket, the running largest abs_diff
 // (and, in a capture segment, the captured values).  Everything else is
 // settled per vector or per item:
 //
-// * tolerance: abs_diff < fma(|gen|, rtol_lo, atol_lo) with both tolerances
-//   lowered by 2^-21 (lean_tol), which never exceeds the exact allowed bound
-//   fl(atol + fl(rtol * |gen|)): such a pair is close (an infinite abs_diff fails);
+// * tolerance: one compare against a bound that never exceeds the exact one
+//   (lean_tol) tells that a pair is close (an infinite abs_diff fails);
 // * rel argmax: best * |ref| >= abs_diff, best the wave's largest rel_diff so
 //   far: such a pair's rel_diff is at most that of an earlier pair;
 // * a pair that fails either test (NaN and Inf do) marks its vector (ballots in
 //   scalar registers, one lane flag per vector); the failing pairs of the
-//   marked vectors go to the queue and slow_elem's exact tests afterwards;
+//   marked vectors go to the queue and slow_elem's exact tests afterwards, except
+//   that most of fp32's mismatches are counted where they are found;
 // * the largest abs_diff is located (lowest index first) only in an item whose
 //   largest exceeds the wave's largest so far;
 // * the ULP distance is the distance of the codes, which is right for pairs of
@@ -1366,24 +1367,6 @@ __device__ __forceinline__ bool phase_b_dense(const SegDesc& d, uint32_t R0, uin
 // behind a branch, a select per ballot and 0.99999 of the largest rel_diff as
 // the bound (which sends every tie to slow_elem), the first two took 158 and
 // 224 us.
-struct LeanTol {
-  float rtol, atol;
-};
-
-// Tolerances for the lean form of the isclose test: fma(|g|, rtol_lo, atol_lo)
-// with x_lo = fl(x * (1 - 2^-21)) <= x * (1 - 2^-22) is at most (X + A) * (1 -
-// 2^-22) before its one rounding, where X = rtol * |g| and A = atol; the exact
-// bound fl(A + fl(X)) is at least (X + A) * (1 - 2^-24) - 2^-150.  For A >=
-// 2^-127 the first is the smaller, and for A = 0 rounding's monotonicity
-// orders them.  Tolerances outside [2^-100, 2^100] (zero aside) or a zero
-// tolerance (plain equality) give bounds below zero: every pair is tested
-// exactly.
-__device__ __forceinline__ LeanTol lean_tol(const SegDesc& d) {
-  auto ok = [](float t) { return t == 0.0f || (t >= 0x1p-100f && t <= 0x1p100f); };
-  if (d.zero_tol || !ok(d.rtol) || !ok(d.atol)) return LeanTol{-1.0f, -1.0f};
-  return LeanTol{d.rtol * (1.0f - 0x1p-21f), d.atol * (1.0f - 0x1p-21f)};
-}
-
 // Absolute difference of two codes (one instruction).
 __device__ __forceinline__ uint32_t abs_diff_u32(uint32_t a, uint32_t b) {
   uint32_t r;
@@ -1442,6 +1425,31 @@ __device__ __forceinline__ void dword_values(uint32_t w, float* f) {
   }
 }
 
+// Whether an item of `pairs` pairs, nq of them slow, is finished as a dense one:
+// dense_pays from one slow pair per lane, each lane's search starting in another
+// vector.
+template <int DT>
+__device__ __forceinline__ bool dense_item(const SegDesc& d, uint64_t slow, uint32_t nq, uint32_t pairs, StageP stage) {
+  using T = typename Elem<DT>::T;
+  constexpr int NE = VecIO<DT>::NE;  // 16 or 32, vector u's first slot at bit u * 4
+  constexpr bool fp32 = DT == KVV_F32;
+  if (dense_surely_pays(fp32, nq, pairs)) return true;
+  const int lane = lane_id(), rot = (lane & 3) * 4;
+  const uint32_t m = (uint32_t)slow;
+  const uint32_t turned = NE == 32 ? __builtin_rotateright32(m, rot) : ((m | (m << 16)) >> rot) & 0xFFFFu;
+  const bool has = turned != 0;
+  int u, e;
+  slot_of<Elem<DT>::width>((int)((has ? __builtin_ctz(turned) : 0) + rot) & (NE - 1), u, e);
+  const float g = Elem<DT>::f32(stage_elem<T>(stage, (2 * u) * 64 + lane, e));
+  const float r = Elem<DT>::f32(stage_elem<T>(stage, (2 * u + 1) * 64 + lane, e));
+  const LeanTol lt = lean_tol(d.rtol, d.atol, d.zero_tol != 0);
+  const float ad = fabsf(g - r);
+  const bool pass = lean_close(ad, g, lt.rtol, lt.atol);
+  return dense_pays(fp32, (d.flags & kFlagCaptureElems) != 0, nq, pairs, (uint32_t)__popcll(ballot(has)),
+                    (uint32_t)__popcll(ballot(has && pass)),
+                    (uint32_t)__popcll(ballot(has && !pass && ad < __builtin_inff())));
+}
+
 // What phase_dense leaves, per lane in the slow-mask layout: the pairs for
 // slow_elem's exact tests, and (NZ, for near_entries) the differing pairs.
 struct DenseLeft {
@@ -1458,7 +1466,7 @@ __device__ __forceinline__ DenseLeft phase_dense(const SegDesc& d, uint32_t R0, 
   constexpr int W = Elem<DT>::width;
   constexpr int EPD = 32 / W;  // elements per dword
   const int lane = lane_id();
-  const LeanTol lt0 = lean_tol(d);
+  const LeanTol lt0 = lean_tol(d.rtol, d.atol, d.zero_tol != 0);
   const float rt = uniform(lt0.rtol);
   float at = lt0.atol;
   asm("" : "+v"(at));  // (in a vector register: an instruction reads one scalar register)
@@ -1516,7 +1524,7 @@ __device__ __forceinline__ DenseLeft phase_dense(const SegDesc& d, uint32_t R0, 
 #pragma unroll
       for (int e = 0; e < EPD; ++e) {
         const float ad = fabsf(g[e] - r[e]);
-        const bool ok = (ad < fmaf(fabsf(g[e]), rt, at)) & (fmaf(thr, fabsf(r[e]), -ad) >= 0.0f);
+        const bool ok = lean_close(ad, g[e], rt, at) & (fmaf(thr, fabsf(r[e]), -ad) >= 0.0f);
         fail |= ballot(!ok);
         im = fmaxf(im, ad);
         const double g64 = (double)g[e], r64 = (double)r[e];
@@ -1604,9 +1612,21 @@ __device__ __forceinline__ DenseLeft phase_dense(const SegDesc& d, uint32_t R0, 
       }
     }
   }
-  // the failing pairs (slow-mask layout), for slow_elem's exact tests
+  // The failing pairs are left (slow-mask layout) for slow_elem's exact tests.  Of
+  // fp32, a finite one whose rel_diff is at most that of an earlier pair and of an
+  // earlier mismatch (the wave's largest) can only be a mismatch: its exact test and
+  // its counts are taken here.
   uint32_t left = 0;
   if (__ballot(fv != 0)) {
+    constexpr bool kHere = DT == KVV_F32;
+    float mthr = -__builtin_inff();
+    if constexpr (kHere) {
+      // (the bound as thr's; no mismatch yet: none is below it)
+      const uint32_t top = wave_max(acc.mm_rel);
+      if (top == 0xFFFFFFFFu) mthr = __builtin_inff();
+      else if (top > (kZeroKey | __float_as_uint(0x1p-40f))) mthr = fkey_value(top);
+      mthr = uniform(mthr);
+    }
 #pragma unroll 1
     for (int u = 0; u < nu; ++u) {
       const bool marked = (fv >> (nu - 1 - u)) & 1u;
@@ -1618,15 +1638,33 @@ __device__ __forceinline__ DenseLeft phase_dense(const SegDesc& d, uint32_t R0, 
 #pragma unroll
         for (int e = 0; e < EPD; ++e) {
           const float ad = fabsf(g[e] - r[e]);
-          const bool ok = (ad < fmaf(fabsf(g[e]), rt, at)) & (fmaf(thr, fabsf(r[e]), -ad) >= 0.0f);
-          left |= (ok ? 0u : 1u) << (e * 16 + u * 4 + j);
+          const bool close = lean_close(ad, g[e], rt, at), low = fmaf(thr, fabsf(r[e]), -ad) >= 0.0f;
+          if constexpr (!kHere) {
+            left |= (close & low ? 0u : 1u) << (e * 16 + u * 4 + j);
+          } else if (!(close & low)) {
+            // (low: abs_diff is finite, and so are both values)
+            if (!close & low & (fmaf(mthr, fabsf(r[e]), -ad) >= 0.0f)) {
+              if (d.zero_tol || !(ad <= d.atol + fabsf(d.rtol * g[e]))) {
+                const uint32_t idx = R0 + (uint32_t)((u * 64 + lane) * V + j), key = __float_as_uint(ad) | kZeroKey;
+                ++acc.nmm;
+                acc.first_mm = idx < acc.first_mm ? idx : acc.first_mm;
+                acc.mm_abs = key > acc.mm_abs ? key : acc.mm_abs;
+              }
+            } else {
+              left |= 1u << (u * 4 + j);
+            }
+          }
         }
       };
       if constexpr (W == 32) {
+        // (one after the other: interleaved, the four took more than 168 registers)
         const uint4 gq = stage_vec(stage, (2 * u) * 64 + lane), rq = stage_vec(stage, (2 * u + 1) * 64 + lane);
         test(gq.x, rq.x, 0);
+        __builtin_amdgcn_sched_barrier(0);
         test(gq.y, rq.y, 1);
+        __builtin_amdgcn_sched_barrier(0);
         test(gq.z, rq.z, 2);
+        __builtin_amdgcn_sched_barrier(0);
         test(gq.w, rq.w, 3);
       } else {
         // (a dword at a time: the vector form took 27 registers more)
@@ -2286,10 +2324,7 @@ __device__ inline void fold_block_record(const LdsRecord* rec, const RunCols& ou
   }
 }
 
-// When the dense path takes an item over from phase A and the queue: a dense
-// item costs about as much as 7 (16-bit) or 3 (fp32) queue steps of 64 slow
-// pairs, i.e. a quarter of the item's.  The kDenseRun items after it skip phase A.
-constexpr uint32_t kDenseShare = 4;
+// Dense items after one that dense_pays chose, without phase A.
 constexpr int kDenseRun = 15;
 
 // ------------------------------------------------------------ scan kernel
@@ -2625,7 +2660,8 @@ __global__ __launch_bounds__(kBlock, BATCH || NZ ? 3 : 1) void scan_kernel(ScanA
             if constexpr (kDense) {
               // (first against the least such item, a constant)
               if (__builtin_expect(nq * kDenseShare >= 64u * VecIO<DT>::V, 0) && dense_fits(full_now, L0, L1) &&
-                  nq * kDenseShare >= (uint32_t)nu * 64u * VecIO<DT>::V) {
+                  nq * kDenseShare >= (uint32_t)nu * 64u * VecIO<DT>::V &&
+                  dense_item<DT>(d, slow, nq, (uint32_t)nu * 64u * VecIO<DT>::V, stage)) {
                 many = true;
                 break;
               }
@@ -2653,14 +2689,17 @@ __global__ __launch_bounds__(kBlock, BATCH || NZ ? 3 : 1) void scan_kernel(ScanA
           for (int k = 0; many; ++k) {
             const DenseLeft o = phase_dense<DT, NZ, BATCH>(d, R0, nu, stage, acc, rep, wc);
             if constexpr (NZ) near_entries<DT>(ni, o.differ, full_now, stage, sink);
+            uint32_t rest = 0;
             if (__ballot(o.test != 0)) {
-              drain(o.test, queue_all<QS>((uint64_t)o.test, sm.queue[w]), [&](uint32_t count) {
+              rest = queue_all<QS>((uint64_t)o.test, sm.queue[w]);
+              drain(o.test, rest, [&](uint32_t count) {
                 phase_b<DT, MODE, true>(d, R0, count, stage, sm.queue[w], acc, wc, rep);
               });
             }
+            const bool more = dense_goes_on(DT == KVV_F32, rest, (uint32_t)nu * 64u * VecIO<DT>::V);
             close_item();
             ++it;
-            many = k < kDenseRun && it < run_end &&
+            many = more && k < kDenseRun && it < run_end &&
                    dense_fits(full, L1, L1 + d.item_elems < d.n ? L1 + d.item_elems : d.n);
             if (many) open_item();
           }

@@ -184,7 +184,7 @@ struct RunCols {
 // sizes[k] (k >= 1) as mulhi(x, mul) >> sh (row_magic).  The loads of such an
 // item waited on up to three 64-bit divisions per lane and vector: a verdict of
 // an 8 x 16 x 1024 x 128 fp16 pair, its reference a permuted view, went from
-// 79 to 72 us; a contiguous pair of that size takes 69.5.  Longer chains of
+// 78.5 to 72.8 us; a contiguous pair of that size takes 69.5.  Longer chains of
 // dims and larger tensors (neither is common) keep the divisions.
 constexpr int kRowDims = 3;
 struct RowMap {
@@ -1361,9 +1361,9 @@ __device__ __forceinline__ bool phase_b_dense(const SegDesc& d, uint32_t R0, uin
 // About 20 instructions per fp32 element (7 of them the fp64 products) and 22
 // per 16-bit element, against the 30 of the earlier in-place fp32 loop and the
 // 100 of phase A, the queue and slow_elem.  Whole verdicts: 8191 x 8191 fp32
-// noise 186 -> 138 us (its loads alone 114), 8192 x 8192 bf16 with half of the
-// pairs one ULP apart under the tolerant policy 315 -> 197 us, the ragged batch
-// of 4,096 pairs 1,365 -> 1,250 us.  With the capture's five tests per element
+// noise 183 -> 136 us (its loads alone 114), 8192 x 8192 bf16 with half of the
+// pairs one ULP apart under the tolerant policy 315 -> 196 us, the ragged batch
+// of 4,096 pairs 1,345 -> 1,242 us.  With the capture's five tests per element
 // behind a branch, a select per ballot and 0.99999 of the largest rel_diff as
 // the bound (which sends every tie to slow_elem), the first two took 158 and
 // 224 us.
